@@ -154,6 +154,7 @@ DeviceCtx* device_ctx() {
         return nullptr;
     }
     c->gqa_lds_ok = attention_device_init();
+    c->prefill_lds_ok = prefill_device_init();
     c->num_cu = cu;
     return c;
 }

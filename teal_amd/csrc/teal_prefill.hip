@@ -14,28 +14,25 @@
 // 9-16 tokens cost 2.1-2.2x the 8-token pass through the module path, profiles/r06_prefill_vs_prompt_length.txt) — the tokens of a
 // feature are one or two 16-byte words (16-bit activations) or KR / 4 of them (fp32 split-K slabs) — so that "row m of every
 // token" is contiguous: a GEMM workgroup
-// stages its slice's rows in LDS once, and a wave then fetches a row with one broadcast read.  The GEMM is bound by HBM like the GEMV (every weight
-// byte is read once for all tokens: 2 * T flops per byte, far from MFMA territory at T <= 8, and the reduction dimension is
-// the strided one in the W^T image, which rules the matrix cores' operand layout out without a second copy of the weights).
+// stages its slice's rows in LDS once, in the matrix cores' operand layout.  The GEMM is bound by HBM like the GEMV (every weight byte is
+// read once for all tokens); its products run on the matrix cores (teal_rows_core.h).
 // Rounding points are those of the module path's 16-bit tensors (projection outputs, RoPE, attention output, residual adds,
 // RMSNorm twice, silu, product); sums are fp32.  Floating-point parity is against the module path, tolerance in the tests.
-#include "teal_common.h"
+#include "teal_rows_core.h"
 
 #include <limits.h>
 
 namespace teal {
 
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kRowsMax = 16;  // most tokens a pass takes; a feature's row holds rows_for(T) of them
 constexpr int kPrefillMaxSplit = 16;
 constexpr int rows_for(const int T) { return T <= 8 ? 8 : 16; }
 
 // sum of `split` slabs in slice order, rounded once to the activation dtype: what a projection's 16-bit output tensor holds
-template <bool BF16, int KR>
+template <bool BF16, int KR, int NT = KR>
 __device__ __forceinline__ void rounded_row(const float* __restrict__ slabs, const int split, const size_t n_total, const size_t col,
-                                            float (&out)[KR]) {
-    constexpr int NW = KR / 4, UU = KR == 8 ? 4 : 2;  // 16-byte words per row; slices whose loads are in flight together
+                                            float (&out)[NT]) {
+    constexpr int NW = NT / 4, UU = NT == 8 ? 4 : 2;  // 16-byte words per row; slices whose loads are in flight together
     f32x4 acc[NW];
 #pragma unroll
     for (int w = 0; w < NW; ++w) acc[w] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -97,180 +94,129 @@ __device__ __forceinline__ void rstd_rows(const float* __restrict__ sumsq, const
 }
 
 // ------------------------------------------------------------------------------------------------
-// slabs[slice][n][8] (fp32) = sum over the slice's rows m of W^T[m][n] * x[token][m], for up to 2 NP tokens.
-//   xt     [Z][8] 16-bit: xt[m][s] = activation m of token s
+// slabs[slice][n][KR] (fp32) = sum over the slice's rows m of W^T[m][n] * x[token][m], for up to KR tokens.
+//   xt     [Z][KR] 16-bit: xt[m][s] = activation m of token s
 //   w0/w1  one or two W^T images [Z][ld]: column tiles < tiles0 stream w0, the others w1 (gate | up in one launch)
-//   grid (256-column tiles, row slices); rows in groups of 16 (one per wave): group q belongs to slice q mod split
-// One WAVE streams one weight row at a time across the whole 256-column tile: 64 lanes x 4 columns = a 512-byte contiguous row
-// segment per load, and the row's activations are WAVE-UNIFORM: the workgroup stages its slice's rows of xt in LDS once and a
-// wave fetches a row's eight tokens with one broadcast LDS read (through scalar loads instead, the loop carried 21 scalar
-// instructions per row — addresses, clamps, selects — and a full `s_waitcnt lgkmcnt(0)` per batch: 3.8 TB/s).  Sixteen rows
-// per wave are in flight (two batches of 8 x 8 bytes per lane: 128 KB per CU, what the GEMV keeps in flight); a lane's sums never
-// leave the lane until the epilogue (no butterflies), where the 16 waves are added in fixed order through LDS, one token pair
-// per round.  Accumulation over pairs of tokens (packed v_pk_fma_f32 until round 6; plain fused multiply-adds since the library
-// is built without packed fp32, profiles/r06_concurrent_packed_fp32.txt: the 6-token pass 4.09 -> 4.25 ms).  First build (row groups inside a wave, the
-// activations through vector loads, 8 rows in flight): 2.1-3.5 TB/s; profiles/r05_prefill_kernel_stats.txt.
+//   grid (128-column tiles, row slices of whole 32-row steps); a step belongs to one of the 8 waves
+// The tokens are one tile of the matrix cores (teal_rows_core.h): the workgroup stages its slice's activations in LDS in their operand
+// layout, eight consecutive features of a token in 16 bytes, and a wave then needs one LDS read, 8 loads and 32 byte permutes per 32 x
+// 128 weights, whatever the number of tokens.
+// Per Llama-2-7B layer (wqkv, wo, w1 | w3, w2; fp16): 7 tokens 30.9 + 13.2 + 48.9 + 28.0 -> 21.1 + 8.7 + 35.4 + 22.2 us, 16 tokens 43.1 + 17.9 +
+// 83.9 + 42.4 -> 27.3 + 9.5 + 43.6 + 28.3 us, against one fused multiply-add per weight and token on the vector ALU (one row per wave
+// and load, 3.3 and 2.1 TB/s).  16 waves instead of 8, or one step in flight per wave instead of two: up to a tenth slower at 16 tokens.
 // ------------------------------------------------------------------------------------------------
-// What the staging loop builds a row's eight activations from (PROD): 0 = xt itself; 1 = RMSNorm of the residual rows ht with the
+// What the staging builds a feature's activations from (PROD): 0 = xt itself; 1 = RMSNorm of the residual rows ht with the
 // per-workgroup sums of squares the resid launch left (every wave adds them itself) and the norm weight; 2 = silu(gate) * up from
 // the slabs of the gate | up launch.  Folding these into the staging removes a launch each: every workgroup builds only the rows
-// of its own slice (a 16th of the vector in the narrow projections), once.
+// of its own slice, once.
 struct PrefillProd {
-    const uint16_t* xt;       // PROD 0: [Z][8];  PROD 1: the residual rows ht [Z][8]
-    const float* sumsq;       // PROD 1: [nwg][8]
+    const uint16_t* xt;       // PROD 0: [Z][KR];  PROD 1: the residual rows ht [Z][KR]
+    const float* sumsq;       // PROD 1: [nwg][KR]
     const uint16_t* norm_w;   // PROD 1: [Z]
-    const float* gu;          // PROD 2: slabs [gu_split][2 Z][8] of the gate | up launch
+    const float* gu;          // PROD 2: slabs [gu_split][2 Z][KR] of the gate | up launch
     float eps;
     int nwg, gu_split, T;
 };
 
-template <bool BF16, int NP, int PROD, int KR>
-__global__ __launch_bounds__(1024) void prefill_gemm_kernel(const PrefillProd pr, const uint16_t* __restrict__ w0, const int ld0,
-                                                            const uint16_t* __restrict__ w1, const int ld1, const int tiles0,
-                                                            float* __restrict__ slabs, const int Z, const int n_total) {
+constexpr int kPrefillWaves = 8, kPrefillTile = 128;
+constexpr int kPrefillSteps = 128;  // most 32-row steps of a slice: 4096 features x 16 tokens x 2 bytes = 128 KB of LDS
+constexpr size_t kPrefillLds = (size_t)kPrefillSteps * 32 * kRowsMax * 2;
+
+// LDS place (16-byte units) of the features 8 kb .. 8 kb + 7 of a token: tokens of neighbouring blocks are turned against each other, so
+// that neither the staging's 4-byte stores nor the operand reads share banks
+template <int KR>
+__device__ __forceinline__ int staged_at(const int kb, const int token) { return kb * KR + (token ^ (kb & (KR - 1))); }
+
+template <bool BF16, int PROD, int KR>
+__global__ __launch_bounds__(64 * kPrefillWaves) void prefill_gemm_kernel(const PrefillProd pr, const uint16_t* __restrict__ w0, const int ld0, const uint16_t* __restrict__ w1,
+                                                                          const int ld1, const int tiles0, float* __restrict__ slabs, const int Z, const int n_total) {
     const uint16_t* __restrict__ xt = pr.xt;
-    // KR = 16 (9-16 tokens): twice the accumulators per lane, so half the weight rows in flight per batch (the loop is bound by
-    // its multiply-adds there, not by the loads) and half the row groups per staging phase (the same 32 KB of activations)
-    constexpr int WAVES = 16, CPL = 4, BN = 256, U = KR == 8 ? 8 : 4, KW = KR / 8, PHASE_GROUPS = 1024 / KR;
-    static_assert(NP <= KR / 2 && NP > (KR == 8 ? 0 : 4), "token pairs of this row width");
     extern __shared__ __align__(16) unsigned char smem[];
-    u32x4* xs = reinterpret_cast<u32x4*>(smem);   // the slice's activation rows of the current phase: xs[(j * 16 + wave) * KW + word]
-    float* red = reinterpret_cast<float*>(smem);  // epilogue (after a barrier): [WAVES][BN][2], one token pair per round
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    u32x4* xs = reinterpret_cast<u32x4*>(smem);   // the slice's activations (staged_at)
+    float* red = reinterpret_cast<float*>(smem);  // epilogue (after a barrier): [wave][column][KR]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
     const int tile = blockIdx.x, slice = blockIdx.y, split = gridDim.y;
     const bool second = tile >= tiles0;
-    const uint32_t ld = (uint32_t)(second ? ld1 : ld0);
-    const int ngroups = Z >> 4;
-    const int nj = (ngroups - slice + split - 1) / split;  // row groups of this slice: q = slice + split * j, row = q * 16 + wave
-    // this wave's rows: base + j * stride (elements)
-    // (a UNIFORM row pointer indexed by the lane: the address is an SGPR base + one 32-bit lane offset, not a 64-bit add per load)
-    const uint16_t* wrow = (second ? w1 : w0) + (size_t)(second ? tile - tiles0 : tile) * BN + (size_t)(slice * 16 + wave) * ld;
-    const size_t stride = (size_t)split * 16u * ld;
-    f32x2 acc[CPL][NP];
+    const int ldb = 2 * (second ? ld1 : ld0), steps = Z >> 5;
+    const int first = (int)((long long)steps * slice / split), n = (int)((long long)steps * (slice + 1) / split) - first;
+    // the slice's rows of the tile's columns; the last row ends with the tile
+    const uint16_t* wb = (second ? w1 : w0) + (size_t)(second ? tile - tiles0 : tile) * kPrefillTile + (size_t)first * 16 * ldb;
+    const RowsBuf buf[1] = {rows_buffer(wb, (size_t)(32 * n - 1) * ldb + 2 * kPrefillTile)};
+    const uint32_t base = (uint32_t)(8 * g) * (uint32_t)ldb + 16u * (uint32_t)l16;
+    auto off = [&](const int s) { return s < n ? base + (uint32_t)s * 32u * (uint32_t)ldb : kRowsNowhere; };
+    RowsTile<8, 1> t0, t1;
+    rows_load<8, 1>(t0, buf, off(wave), ldb);
+    [[maybe_unused]] float rstd[KR];
+    if constexpr (PROD == 1) rstd_rows<KR>(pr.sumsq, pr.nwg, lane, Z, pr.eps, rstd);
+    // a thread and round: two features of eight tokens
+    for (int u = tid; u < n * 16 * (KR / 8); u += 64 * kPrefillWaves) {
+        const int o8 = KR == 8 ? 0 : 8 * (u & 1), pair = KR == 8 ? u : u >> 1;
+        const uint32_t m0 = (uint32_t)first * 32u + 2u * (uint32_t)pair;
+        uint32_t word[8];  // per token: features m0, m0 + 1
+        if constexpr (PROD == 0) {
+            const u32x4 a = *reinterpret_cast<const u32x4*>(xt + (size_t)m0 * KR + o8), b = *reinterpret_cast<const u32x4*>(xt + (size_t)(m0 + 1) * KR + o8);
 #pragma unroll
-    for (int c = 0; c < CPL; ++c)
-#pragma unroll
-        for (int p = 0; p < NP; ++p) acc[c][p] = (f32x2){0.0f, 0.0f};
-    auto consume = [&](const u32x2 w, const u32x4 (&xv)[KW]) {
-        f32x2 xp[NP];
-#pragma unroll
-        for (int p = 0; p < NP; ++p) xp[p] = (f32x2){bits_to_float(xv[p >> 2][p & 3] & 0xFFFFu, BF16), bits_to_float(xv[p >> 2][p & 3] >> 16, BF16)};
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const float wl = bits_to_float(w[j] & 0xFFFFu, BF16), wh = bits_to_float(w[j] >> 16, BF16);
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                acc[2 * j][p] = __builtin_elementwise_fma((f32x2){wl, wl}, xp[p], acc[2 * j][p]);
-                acc[2 * j + 1][p] = __builtin_elementwise_fma((f32x2){wh, wh}, xp[p], acc[2 * j + 1][p]);
+            for (int d = 0; d < 4; ++d) {
+                word[2 * d] = __builtin_amdgcn_perm(b[d], a[d], 0x05040100u);
+                word[2 * d + 1] = __builtin_amdgcn_perm(b[d], a[d], 0x07060302u);
             }
-        }
-    };
-    for (int jb = 0; jb < nj; jb += PHASE_GROUPS) {
-        const int njp = min(PHASE_GROUPS, nj - jb);  // groups of this phase (one phase for every Llama-2-7B launch)
-        const uint16_t* wph = wrow + (size_t)jb * stride;
-        const int nfull = njp / (2 * U);  // whole pairs of batches
-        // (staging the rows as fp32 — no conversion of the activations in the loop: 17 instead of 25 vector instructions per row —
-        //  was measured too: no faster, gate | up 41.3 -> 43.6 us: the loop is not bound by its conversions)
-        // (requesting the first batch of weight rows ahead of the staging — nothing in it depends on the activations — was
-        //  measured: the 16 registers it keeps live through the producers push the kernel to 126-128 registers with spills, and
-        //  the gate | up launch went 41 -> 48 us; profiles/r05_prefill_kernel_stats.txt)
-        if (jb) __syncthreads();
-        [[maybe_unused]] float rstd[KR];
-        if constexpr (PROD == 1) rstd_rows<KR>(pr.sumsq, pr.nwg, lane, Z, pr.eps, rstd);
-        for (int r = tid; r < njp * 16; r += 1024) {
-            const uint32_t m = (uint32_t)(slice + split * (jb + (r >> 4))) * 16u + (uint32_t)(r & 15);
-            [[maybe_unused]] uint16_t* dst = reinterpret_cast<uint16_t*>(xs + (size_t)r * KW);
-            if constexpr (PROD == 0) {
+        } else {
 #pragma unroll
-                for (int w = 0; w < KW; ++w) xs[(size_t)r * KW + w] = *reinterpret_cast<const u32x4*>(xt + (size_t)m * KR + 8 * w);
-            } else if constexpr (PROD == 1) {  // x = round(round(h * rstd) * w)  (gpt-fast/model.py:289-291)
-                const float nw = bits_to_float(pr.norm_w[m], BF16);
-                float x[KR];
-                load_row<BF16, KR>(xt + (size_t)m * KR, x);
+            for (int e = 0; e < 2; ++e) {
+                const uint32_t m = m0 + e;
+                float x[8];
+                if constexpr (PROD == 1) {  // x = round(round(h * rstd) * w)  (gpt-fast/model.py:289-291)
+                    const float nw = bits_to_float(pr.norm_w[m], BF16);
+                    load_row<BF16, 8>(xt + (size_t)m * KR + o8, x);
 #pragma unroll
-                for (int s_ = 0; s_ < KR; ++s_) {
-                    const float xn = bits_to_float(float_to_bits<BF16>(x[s_] * rstd[s_]), BF16);
-                    x[s_] = s_ < pr.T ? bits_to_float(float_to_bits<BF16>(xn * nw), BF16) : 0.0f;
+                    for (int s = 0; s < 8; ++s) x[s] = bits_to_float(float_to_bits<BF16>(x[s] * (KR == 8 || !o8 ? rstd[s] : rstd[KR - 8 + s])), BF16) * nw;
+                } else {  // x = round(round(silu(round(gate))) * round(up))  (gpt-fast/model.py:258-259)
+                    float gv[8], uv[8];
+                    rounded_row<BF16, KR, 8>(pr.gu + o8, pr.gu_split, (size_t)2 * Z, (size_t)m, gv);
+                    rounded_row<BF16, KR, 8>(pr.gu + o8, pr.gu_split, (size_t)2 * Z, (size_t)Z + m, uv);
+#pragma unroll
+                    for (int s = 0; s < 8; ++s) x[s] = bits_to_float(float_to_bits<BF16>(gv[s] / (1.0f + expf(-gv[s]))), BF16) * uv[s];
                 }
-                store_row<BF16, KR>(dst, x);
-            } else {  // x = round(round(silu(round(gate))) * round(up))  (gpt-fast/model.py:258-259)
-                float gv[KR], uv[KR], x[KR];
-                rounded_row<BF16, KR>(pr.gu, pr.gu_split, (size_t)2 * Z, (size_t)m, gv);
-                rounded_row<BF16, KR>(pr.gu, pr.gu_split, (size_t)2 * Z, (size_t)Z + m, uv);
 #pragma unroll
-                for (int s_ = 0; s_ < KR; ++s_) {
-                    const float sl = bits_to_float(float_to_bits<BF16>(gv[s_] / (1.0f + expf(-gv[s_]))), BF16);
-                    x[s_] = s_ < pr.T ? bits_to_float(float_to_bits<BF16>(sl * uv[s_]), BF16) : 0.0f;
+                for (int s = 0; s < 8; ++s) {
+                    const uint32_t b = o8 + s < pr.T ? float_to_bits<BF16>(x[s]) : 0u;
+                    word[s] = e ? word[s] | (b << 16) : b;
                 }
-                store_row<BF16, KR>(dst, x);
             }
         }
-        __syncthreads();
-        // rows past the phase's last group (GUARD: only the last, partial pair of batches) repeat it; their activations read as zero
-        auto issue = [&](u32x2 (&w)[U], const int j0, auto guard) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int j = decltype(guard)::value ? min(j0 + u, njp - 1) : j0 + u;
-                w[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(wph + (size_t)j * stride) + (uint32_t)lane);
-            }
-        };
-        auto consume_batch = [&](const u32x2 (&w)[U], const int j0, auto guard) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int j = decltype(guard)::value ? min(j0 + u, njp - 1) : j0 + u;
-                u32x4 xv[KW];
-#pragma unroll
-                for (int q = 0; q < KW; ++q) {
-                    xv[q] = xs[(j * 16 + wave) * KW + q];  // wave-uniform address: one LDS broadcast read per word
-                    if (decltype(guard)::value && j0 + u >= njp) xv[q] = (u32x4){0u, 0u, 0u, 0u};
-                }
-                consume(w[u], xv);
-            }
-        };
-        // software pipeline, two batches of U rows in flight (scheduling barriers: left alone, the machine scheduler sinks every
-        // load to just above its first use to save registers — one load in flight per wave and an `s_waitcnt vmcnt(0)` per row)
-        constexpr std::false_type full{};
-        constexpr std::true_type guarded{};
-        u32x2 wa[U], wb[U];
-        int j0 = 0;
-        if (nfull > 0) {
-            issue(wa, 0, full);
-            __builtin_amdgcn_sched_barrier(0);
-            for (int it = 0; it < nfull; ++it, j0 += 2 * U) {
-                issue(wb, j0 + U, full);
-                __builtin_amdgcn_sched_barrier(0);
-                consume_batch(wa, j0, full);
-                __builtin_amdgcn_sched_barrier(0);
-                if (it + 1 < nfull) issue(wa, j0 + 2 * U, full);
-                __builtin_amdgcn_sched_barrier(0);
-                consume_batch(wb, j0 + U, full);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        if (j0 < njp) {  // the partial pair: one guarded batch if U rows or fewer remain, else two
-            issue(wa, j0, guarded);
-            const bool two = j0 + U < njp;
-            if (two) issue(wb, j0 + U, guarded);
-            __builtin_amdgcn_sched_barrier(0);
-            consume_batch(wa, j0, guarded);
-            if (two) consume_batch(wb, j0 + U, guarded);
-        }
+        for (int s = 0; s < 8; ++s) reinterpret_cast<uint32_t*>(xs + staged_at<KR>(pair >> 2, o8 + s))[pair & 3] = word[s];
     }
-    // the 16 waves in fixed order through LDS, one token pair per round
-    const uint32_t col_base = (uint32_t)tile * BN;
+    rows_load<8, 1>(t1, buf, off(wave + kPrefillWaves), ldb);
+    f32x4 acc[1][8];
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-        __syncthreads();
+    for (int f = 0; f < 8; ++f) acc[0][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+    auto product = [&](const RowsTile<8, 1>& t, const int s) {
+        const u32x4 x[1] = {xs[staged_at<KR>(4 * s + g, l16 & (KR - 1))]};
+        rows_mfma<BF16, true, 1, 8, 1>(t, x, acc);
+    };
+    int s = wave;
+    for (; s + kPrefillWaves < n; s += 2 * kPrefillWaves) {
+        product(t0, s);
+        rows_load<8, 1>(t0, buf, off(s + 2 * kPrefillWaves), ldb);
+        product(t1, s + kPrefillWaves);
+        rows_load<8, 1>(t1, buf, off(s + 3 * kPrefillWaves), ldb);
+    }
+    if (s < n) product(t0, s);
+    // the waves in fixed order through LDS; column 8 * l16 + f of the tile is stored at f * 16 + l16 (a wave's stores are contiguous)
+    __syncthreads();
+    if (KR == 16 || g < 2) {
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) *reinterpret_cast<f32x2*>(red + ((size_t)wave * BN + lane * CPL + c) * 2) = acc[c][p];
-        __syncthreads();
-        if (tid < BN * 2) {
-            const int col = tid >> 1, e = tid & 1;
-            float sum = 0.0f;
+        for (int f = 0; f < 8; ++f) *reinterpret_cast<f32x4*>(red + ((size_t)wave * kPrefillTile + f * 16 + l16) * KR + 4 * g) = acc[0][f];
+    }
+    __syncthreads();
+    if (tid < kPrefillTile * KR / 4) {
+        const int p = tid / (KR / 4), q = tid % (KR / 4), col = 8 * (p & 15) + (p >> 4);
+        f32x4 sum = *reinterpret_cast<const f32x4*>(red + (size_t)p * KR + 4 * q);
 #pragma unroll
-            for (int w = 0; w < WAVES; ++w) sum += red[((size_t)w * BN + col) * 2 + e];
-            slabs[((size_t)slice * n_total + col_base + col) * KR + 2 * p + e] = sum;
-        }
+        for (int w = 1; w < kPrefillWaves; ++w) sum += *reinterpret_cast<const f32x4*>(red + ((size_t)w * kPrefillTile + p) * KR + 4 * q);
+        *reinterpret_cast<f32x4*>(slabs + ((size_t)slice * n_total + (size_t)tile * kPrefillTile + col) * KR + 4 * q) = sum;
     }
 }
 
@@ -449,6 +395,19 @@ __global__ __launch_bounds__(HD) void prefill_attention_kernel(const float* __re
     store_row<BF16, KR>(yt + ((size_t)h * HD + d) * KR, o);
 }
 
+bool prefill_device_init() {
+    bool ok = true;
+#define TEAL_OPT(BF, KRV) do { \
+        ok = ok && hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_kernel<BF, 0, KRV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPrefillLds) == hipSuccess; \
+        ok = ok && hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_kernel<BF, 1, KRV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPrefillLds) == hipSuccess; \
+        ok = ok && hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_kernel<BF, 2, KRV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kPrefillLds) == hipSuccess; \
+    } while (0)
+    TEAL_OPT(false, 8); TEAL_OPT(false, 16); TEAL_OPT(true, 8); TEAL_OPT(true, 16);
+#undef TEAL_OPT
+    if (!ok) (void)hipGetLastError();
+    return ok;
+}
+
 }  // namespace teal
 
 using namespace teal;
@@ -482,37 +441,33 @@ int teal_prefill_gemm(const teal_prefill_in_t* in, const void* w0T, int ld0, int
     }
     if (!aligned16(w0T) || (w1T && !aligned16(w1T)) || !aligned16(slabs)) return TEAL_ERR_ALIGN;
     DeviceCtx* ctx = device_ctx();
-    if (!ctx) return TEAL_ERR_NO_DEVICE;
+    if (!ctx || !ctx->prefill_lds_ok) return TEAL_ERR_NO_DEVICE;
     const int ncu = ctx->num_cu, ntot = n0 + n1;
-    // 256-column tiles; the 16-row groups are dealt to `split` slices: never more workgroups than CUs (a 16-wave workgroup owns its
-    // CU: 86 tiles x 3 = 258 workgroups ran 62 us, x 2 = 172 run 38), every wave keeping at least one full pair of batches
-    // (split <= Z / 256), and among the candidates the one whose waves stream the fewest 8-row batches (ties: the fewer slabs)
-    constexpr int bn = 256;
-    if (n0 % bn || n1 % bn) return TEAL_ERR_SHAPE;
-    const int tiles = ntot / bn, ngroups = Z >> 4;
+    // 128-column tiles; whole 32-row steps are dealt to `split` slices: never more workgroups than CUs (the staged activations take its LDS), a
+    // step per wave at least, a slice's activations within the LDS, and among the candidates the one whose waves take the fewest steps (ties:
+    // the fewer slabs)
+    if (n0 % 256 || n1 % 256) return TEAL_ERR_SHAPE;
+    const int tiles = ntot / kPrefillTile, steps = Z >> 5, smin = (steps + kPrefillSteps - 1) / kPrefillSteps;
     int smax = ncu / tiles;
-    if (smax > Z / 256) smax = Z / 256;
+    if (smax > steps / kPrefillWaves) smax = steps / kPrefillWaves;
     if (smax > kPrefillMaxSplit) smax = kPrefillMaxSplit;
-    if (smax < 1) smax = 1;
-    int split = 1, best = INT_MAX;
-    for (int c = 1; c <= smax; ++c) {
-        const int batches = ((ngroups + c - 1) / c + 7) / 8;
-        if (batches < best) { best = batches; split = c; }
+    int split = smin, best = INT_MAX;
+    for (int c = smin; c <= smax; ++c) {
+        const int rounds = ((steps + c - 1) / c + kPrefillWaves - 1) / kPrefillWaves;
+        if (rounds < best) { best = rounds; split = c; }
     }
     if (slabs_bytes < (size_t)split * ntot * kr * sizeof(float)) return TEAL_ERR_WORKSPACE;
-    const dim3 grid(tiles, split), block(1024);
-    const size_t lds = (size_t)16 * bn * 2 * sizeof(float);  // 32 KB: the activation rows of a phase, then the reduction tile
+    const dim3 grid(tiles, split), block(64 * kPrefillWaves);
+    const size_t staged = (size_t)((steps + split - 1) / split) * 32 * kr * 2, reduced = (size_t)kPrefillWaves * kPrefillTile * kr * sizeof(float);
+    const size_t lds = staged > reduced ? staged : reduced;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const int np = (T + 1) / 2, tiles0 = n0 / bn;
+    const int tiles0 = n0 / kPrefillTile;
     auto* a = reinterpret_cast<const uint16_t*>(w0T);
     auto* b = reinterpret_cast<const uint16_t*>(w1T);
-#define TEAL_PG(BF, NPV, PR, KRV) hipLaunchKernelGGL((prefill_gemm_kernel<BF, NPV, PR, KRV>), grid, block, lds, st, pr, a, ld0, b, ld1, tiles0, slabs, Z, ntot)
-#define TEAL_PG_PR(BF, NPV, KRV) do { if (in->mode == TEAL_PREFILL_IN_NORM) TEAL_PG(BF, NPV, 1, KRV); else if (in->mode == TEAL_PREFILL_IN_SILU_MUL) TEAL_PG(BF, NPV, 2, KRV); else TEAL_PG(BF, NPV, 0, KRV); } while (0)
-#define TEAL_PG_NP(BF) do { switch (np) { case 1: TEAL_PG_PR(BF, 1, 8); break; case 2: TEAL_PG_PR(BF, 2, 8); break; case 3: TEAL_PG_PR(BF, 3, 8); break; \
-    case 4: TEAL_PG_PR(BF, 4, 8); break; case 5: TEAL_PG_PR(BF, 5, 16); break; case 6: TEAL_PG_PR(BF, 6, 16); break; case 7: TEAL_PG_PR(BF, 7, 16); break; \
-    default: TEAL_PG_PR(BF, 8, 16); } } while (0)
-    if (dtype == TEAL_BF16) TEAL_PG_NP(true); else TEAL_PG_NP(false);
-#undef TEAL_PG_NP
+#define TEAL_PG(BF, PR, KRV) hipLaunchKernelGGL((prefill_gemm_kernel<BF, PR, KRV>), grid, block, lds, st, pr, a, ld0, b, ld1, tiles0, slabs, Z, ntot)
+#define TEAL_PG_PR(BF, KRV) do { if (in->mode == TEAL_PREFILL_IN_NORM) TEAL_PG(BF, 1, KRV); else if (in->mode == TEAL_PREFILL_IN_SILU_MUL) TEAL_PG(BF, 2, KRV); else TEAL_PG(BF, 0, KRV); } while (0)
+    if (dtype == TEAL_BF16) { if (kr == 8) TEAL_PG_PR(true, 8); else TEAL_PG_PR(true, 16); }
+    else { if (kr == 8) TEAL_PG_PR(false, 8); else TEAL_PG_PR(false, 16); }
 #undef TEAL_PG_PR
 #undef TEAL_PG
     *split_out = split;
