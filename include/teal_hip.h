@@ -399,6 +399,33 @@ int teal_prefill_resid_norm(const void* emb, const int32_t* tokens, int T, const
 int teal_prefill_attention(const float* qkv_slabs, int split, const void* rope, void* k_cache, void* v_cache, void* yt, int T, int n_head,
                            int n_kv_head, int head_dim, int max_seq, int dtype, void* stream);
 
+/* ---- matrix products over a few rows, teal_amd/csrc/teal_rows.hip -----------------------------------------------------
+ * y[M][N] = x[M][K] * W^T image [K][ld] for M <= 64, K % 32 == 0, N % 8 == 0, 16-bit operands, fp32 sums (over slices of K in slice order:
+ * bit-reproducible).  x rows ldx apart (ldx % 8 == 0), ld % 8 == 0; x, images and biases 16-byte aligned. */
+#define TEAL_ROWS_ROUNDED 0 /* y 16-bit [M][ldy] (ldy % 4 == 0) = round(act(sum + bias)), or with w_up round(act(sum + bias) * (sum_up + bias_up)) */
+#define TEAL_ROWS_SLABS 1   /* y fp32 [teal_rows_split()][M][N]: the slices' partial sums, for the consumer to add in slice order */
+#define TEAL_ROWS_F32 2     /* y fp32 [M][ldy], columns < n_valid: the sum, or softcap * tanh(sum / softcap) */
+#define TEAL_ACT_NONE (-1)
+#define TEAL_ACT_SILU_ROUNDED 3 /* with w_up: round(silu(round(gate))) * round(up), the rounding points of gpt-fast/model.py:258-259 */
+typedef struct teal_rows_gemm {
+    const void* x;
+    const void* w;
+    const void* w_up;          /* optional second image (same ld): gate = w, up = w_up */
+    const void* bias;          /* optional, 16-bit [N] */
+    const void* bias_up;
+    void* y;
+    float* part;               /* ROUNDED, F32 when teal_rows_split() > 1: scratch, split * M * (N rounded up to 128, with w_up 2 N to 128) floats */
+    size_t part_bytes;
+    unsigned* tickets;         /* ... and one zero counter per 128 (with w_up 64) columns, <= 256; zero again afterwards.  Launches that may
+                                * overlap need their own */
+    int M, K, N, ldx, ld, ldy;
+    int mode, act, n_valid;
+    float softcap;
+} teal_rows_gemm_t;
+/* slices a launch of this shape takes (>= 1); 0: outside the kernel's shapes */
+int teal_rows_split(int M, int K, int N, int paired);
+int teal_rows_gemm(const teal_rows_gemm_t* args, int dtype, void* stream);
+
 /* ---- layered decoder designs: row kernels around their matrix products, teal_amd/csrc/teal_layered.hip ----------------
  * dtype 0 / 1 / 2 (fp16, bf16, fp32) = activations and weights; the residual stream is always fp32. */
 
@@ -408,6 +435,11 @@ int teal_prefill_attention(const float* qkv_slabs, int split, const void* rope, 
 int teal_layer_resid_norm(float* x, int n_rows, int dim, const int32_t* tokens, const void* embed, int vocab, const void* y, int ldy,
                           const void* y_bias, const void* post_w, const void* pre_w, float norm_offset, float eps, void* h,
                           const int32_t* rows, int dtype, void* stream);
+/* the same with y = the sum of n_slabs fp32 slabs [n_slabs][n_rows][ldy] in slab order (TEAL_ROWS_SLABS; rows: indexes them too, of slab_rows
+ * rows); zero: optional, n_zero <= 256 counters set to zero (the tickets of the products that follow) */
+int teal_layer_resid_norm_slabs(float* x, int n_rows, int dim, const int32_t* tokens, const void* embed, int vocab, const float* y, int n_slabs, int slab_rows,
+                                int ldy, const void* y_bias, const void* post_w, const void* pre_w, float norm_offset, float eps, void* h,
+                                const int32_t* rows, unsigned* zero, int n_zero, int dtype, void* stream);
 #define TEAL_ACT_SILU 0
 #define TEAL_ACT_GELU_TANH 1
 #define TEAL_ACT_RELU2 2 /* max(z, 0)^2 */

@@ -21,6 +21,9 @@ struct ResidNormArgs {
     const int32_t* rows;    // or null: row of x / y / tokens a workgroup handles (a subset of the rows); h is packed
     int D, ldy, vocab;
     float eps, off;         // off: added to the norms' weights (weights stored around zero: 1)
+    int nslabs, slab_rows;  // nslabs > 0: y is the sum of fp32 slabs [nslabs][slab_rows][ldy]
+    unsigned* zero;         // or null: nzero counters to clear
+    int nzero;
 };
 
 template <int DT, int NT, int VEC>
@@ -32,7 +35,9 @@ __global__ __launch_bounds__(NT) void resid_norm_kernel(const ResidNormArgs a) {
     __shared__ float red[NT / 64];
     const int tid = threadIdx.x, D = a.D;
     const size_t row = a.rows ? (size_t)a.rows[blockIdx.x] : (size_t)blockIdx.x;
+    if (blockIdx.x == 0 && tid < a.nzero) a.zero[tid] = 0u;
     float* x = a.x + row * D;
+    const float* ys = reinterpret_cast<const float*>(a.y) + row * a.ldy;
     const S* y = a.y ? reinterpret_cast<const S*>(a.y) + row * a.ldy : nullptr;
     const S* yb = reinterpret_cast<const S*>(a.y_bias);
     const S* pw = reinterpret_cast<const S*>(a.post_w);
@@ -68,7 +73,17 @@ __global__ __launch_bounds__(NT) void resid_norm_kernel(const ResidNormArgs a) {
         float ss = 0.0f;
         for (int i = tid * VEC; i < D; i += NT * VEC) {
             float v[VEC];
-            ldv(y + i, v);
+            if (a.nslabs) {
+                ldx(ys + i, v);
+                for (int k = 1; k < a.nslabs; ++k) {
+                    float u[VEC];
+                    ldx(ys + (size_t)k * a.slab_rows * a.ldy + i, u);
+#pragma unroll
+                    for (int j = 0; j < VEC; ++j) v[j] += u[j];
+                }
+            } else {
+                ldv(y + i, v);
+            }
             if (yb) {
                 float b[VEC];
                 ldv(yb + i, b);
@@ -293,27 +308,39 @@ using namespace teal;
 
 extern "C" {
 
-int teal_layer_resid_norm(float* x, int n_rows, int dim, const int32_t* tokens, const void* embed, int vocab, const void* y, int ldy,
-                          const void* y_bias, const void* post_w, const void* pre_w, float norm_offset, float eps, void* h, const int32_t* rows, int dtype,
-                          void* stream) {
-    if (!x || n_rows <= 0 || dim <= 0 || (tokens && (!embed || vocab <= 0)) || (post_w && !y) || (y_bias && !y) || (pre_w && !h)) return TEAL_ERR_ARG;
-    if (dim > 15360 || (y && ldy < dim)) return TEAL_ERR_SHAPE;
+static int resid_norm_launch(const ResidNormArgs& a, int n_rows, int dtype, void* stream) {
+    const bool y = a.y != nullptr;
+    if (!a.x || n_rows <= 0 || a.D <= 0 || (a.tokens && (!a.embed || a.vocab <= 0)) || (a.post_w && !y) || (a.y_bias && !y) || (a.pre_w && !a.h)) return TEAL_ERR_ARG;
+    if (a.D > 15360 || (y && a.ldy < a.D)) return TEAL_ERR_SHAPE;
     if (!device_ctx()) return TEAL_ERR_NO_DEVICE;
-    const ResidNormArgs a = {x, tokens, embed, y, y_bias, post_w, pre_w, h, rows, dim, ldy, vocab, eps, norm_offset};
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const void* ps[] = {x, embed, y, y_bias, post_w, pre_w, h};
-    bool vec = (dim & 3) == 0 && (!y || (ldy & 3) == 0);
+    const void* ps[] = {a.x, a.embed, a.y, a.y_bias, a.post_w, a.pre_w, a.h};
+    bool vec = (a.D & 3) == 0 && (!y || (a.ldy & 3) == 0);
     for (const void* p : ps) vec = vec && aligned16(p);
     return with_dtype(dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
-        const size_t lds = (size_t)dim * sizeof(float);
+        const size_t lds = (size_t)a.D * sizeof(float);
 #define TEAL_RN(NT, V) hipLaunchKernelGGL((resid_norm_kernel<DT, NT, V>), dim3(n_rows), dim3(NT), lds, st, a)
         if (!vec) TEAL_RN(256, 1);
-        else if (dim <= 2048) TEAL_RN(256, 4);
+        else if (a.D <= 2048) TEAL_RN(256, 4);
         else TEAL_RN(1024, 4);
 #undef TEAL_RN
         return launched();
     });
+}
+
+int teal_layer_resid_norm(float* x, int n_rows, int dim, const int32_t* tokens, const void* embed, int vocab, const void* y, int ldy,
+                          const void* y_bias, const void* post_w, const void* pre_w, float norm_offset, float eps, void* h, const int32_t* rows, int dtype,
+                          void* stream) {
+    return resid_norm_launch({x, tokens, embed, y, y_bias, post_w, pre_w, h, rows, dim, ldy, vocab, eps, norm_offset, 0, 0, nullptr, 0}, n_rows, dtype, stream);
+}
+
+int teal_layer_resid_norm_slabs(float* x, int n_rows, int dim, const int32_t* tokens, const void* embed, int vocab, const float* y, int n_slabs, int slab_rows,
+                                int ldy, const void* y_bias, const void* post_w, const void* pre_w, float norm_offset, float eps, void* h,
+                                const int32_t* rows, unsigned* zero, int n_zero, int dtype, void* stream) {
+    if ((y && (n_slabs < 1 || slab_rows < 1)) || (zero && (n_zero < 1 || n_zero > 256))) return TEAL_ERR_ARG;
+    return resid_norm_launch({x, tokens, embed, y, y_bias, post_w, pre_w, h, rows, dim, ldy, vocab, eps, norm_offset, y ? n_slabs : 0, slab_rows, zero, zero ? n_zero : 0},
+                             n_rows, dtype, stream);
 }
 
 int teal_gated_act(const void* gu, int ldg, int up0, const void* bias_gate, const void* bias_up, void* h, int ldh, int n_rows, int n_cols, int act,

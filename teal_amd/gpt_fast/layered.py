@@ -9,8 +9,8 @@ Designs: Bolizen (latent attention) and Tefopel (time mixing with a recurrent st
 use another layer's weights).
 
 Two passes share one set of weights and one cache (paged.PagedCache: pages of rows, recurrent states per slot):
-  prompt pass   ragged batch of portions (each any number of tokens, from any position), packed without padding; matrix products by
-                the vendor library over MFMA, hand-written kernels for everything between them (csrc/teal_layered.hip, teal_latent.hip,
+  prompt pass   ragged batch of portions (each any number of tokens, from any position), packed without padding; matrix products over a
+                few rows by teal_rows.hip, larger ones by the vendor library, hand-written kernels for everything between them (csrc/teal_layered.hip, teal_latent.hip,
                 teal_grouped.hip, teal_wkv.hip)
   step          one token per sequence; attention over the cached rows as they are, recurrences by one token
 The residual stream is fp32 throughout.  dtype fp16 / bf16 (matrix products and activations) or float32 (everything).
@@ -294,6 +294,7 @@ class PromptBatch:
         self.key_row = dev[5 * q0:5 * q0 + k0]
         self.seqs = dev[5 * q0 + k0:].view(-1, 5)
         self.device = device
+        self.tickets: Optional[torch.Tensor] = None  # counters of the running pass (LayeredTransformer._run)
         self._tiles: Dict[int, torch.Tensor] = {}
         self.packed: Dict[int, Any] = {}  # owner layer -> (latents, rotated key parts) of every key row of the batch
 
@@ -322,6 +323,7 @@ class StepBatch:
     pos: torch.Tensor
     slot: torch.Tensor
     max_pos: int                     # no position of the batch is larger (chooses how far the attention is split; not a limit)
+    tickets: Optional[torch.Tensor] = None  # counters of the running pass (LayeredTransformer._run)
 
 
 # ------------------------------------------------------------------------------------------------
@@ -419,7 +421,7 @@ class LatentAttention(nn.Module):
         a, owner = self.a, self.owner(index)
         pool = b.cache.pools[owner]
         own = a.kv_from is None
-        proj = self.proj(h)
+        proj = K.linear(self.proj, h, b.tickets)
         K.latent_prompt_rows(proj, self.kv0 if own else -1, b.pos, b.row if own else None, self.inv_freq, self.kv_norm, self.eps, a.heads, a.dim, a.rot_dim,
                              a.kv_rank, pool if own else None)
         if own:
@@ -429,7 +431,7 @@ class LatentAttention(nn.Module):
         tile = self.prompt_tile(b)
         y = K.prompt_attention(proj, k, kr, vt, self.sink, self._gate(proj), padded_rows(b.n_tokens, self.nv, self.wo, h), b.seqs, b.tiles(tile), tile, a.heads, a.dim,
                                       a.rot_dim, a.vdim, self.window, a.scale)
-        return self.wo(y)
+        return K.linear(self.wo, y, b.tickets, slabs=True)
 
     def splits(self, batch: int, max_pos: int, dtype: torch.dtype) -> int:
         """workgroups the cached rows of one sequence are split over: two per CU in all, one 32-key tile each at least"""
@@ -457,7 +459,7 @@ class LatentAttention(nn.Module):
         return K.latent_step_merge(part, splits, self.uv, self.sink, self._gate(proj), y, n, a.heads, a.kv_rank, a.vdim)
 
     def step(self, h: torch.Tensor, b: StepBatch, index: Optional[int] = None) -> torch.Tensor:
-        return self.wo(self.attend(self.proj(h), b, index=index))
+        return K.linear(self.wo, self.attend(K.linear(self.proj, h, b.tickets), b, index=index), b.tickets, slabs=True)
 
     def linears(self):
         return [self.proj, self.wo]
@@ -530,13 +532,13 @@ class GroupedAttention(nn.Module):
 
     def prompt(self, h: torch.Tensor, b: PromptBatch, index: Optional[int] = None) -> torch.Tensor:
         a, pool = self.a, b.cache.pools[self.owner(index)]
-        proj = self.proj(h)
+        proj = K.linear(self.proj, h, b.tickets)
         K.grouped_prompt_rows(proj, self.k0, b.pos, b.row, self.inv_freq, a.heads, a.kv_heads, a.dim, a.rot_dims, pool)
         k, vt = K.grouped_gather(pool, b.key_row, a.kv_heads, a.dim, a.rot_dims)
         tile = self.prompt_tile(b)
         y = K.prompt_attention(proj, k, None, vt, self.sink, None, padded_rows(b.n_tokens, self.nv, self.wo, h), b.seqs, b.tiles(tile), tile, a.heads, a.dim, 0, a.dim,
                                self.window, a.scale, self.group, a.softcap)
-        return self.wo(y)
+        return K.linear(self.wo, y, b.tickets, slabs=True)
 
     def splits(self, batch: int, max_pos: int, dtype: torch.dtype) -> int:
         groups = self.a.heads if dtype == torch.float32 else self.a.kv_heads * -(-self.group // 16)
@@ -561,7 +563,7 @@ class GroupedAttention(nn.Module):
         return K.grouped_step_merge(part, splits, self.sink, y, n, a.heads, a.dim)
 
     def step(self, h: torch.Tensor, b: StepBatch, index: Optional[int] = None) -> torch.Tensor:
-        return self.wo(self.attend(self.proj(h), b, index=index))
+        return K.linear(self.wo, self.attend(K.linear(self.proj, h, b.tickets), b, index=index), b.tickets, slabs=True)
 
     def linears(self):
         return [self.proj, self.wo]
@@ -631,13 +633,13 @@ class TimeMix(nn.Module):
         """-> r, k, v, g [rows, heads * dim], z [rows, rank]"""
         mixes = self.mixed(K.wkv_mix(x, norm_w, self.norm_offset, self.eps, self.mu, b.pos, b.slot, run, b.cache.states[self.owner(index), "shift"]))
         w, n = self.proj.weight, (self.nv,) * 4 + (self.a.decay_rank,)
-        return [nn.functional.linear(mixes[i], w[i * self.seg:i * self.seg + n[i]]) for i in range(5)]
+        return [K.linear(None, mixes[i], b.tickets, weight=w[i * self.seg:i * self.seg + n[i]]) for i in range(5)]
 
     def prompt(self, x: torch.Tensor, norm_w: torch.Tensor, b: PromptBatch, index: Optional[int] = None) -> torch.Tensor:
         a = self.a
         r, k, v, g, z = self._project(x, norm_w, b, b.run, index)
         o = K.wkv_scan(r, k, v, K.wkv_decay(z, self.w2, self.w0), self.u, b.seqs, b.slot, b.cache.states[self.owner(index), "wkv"], b.longest)
-        return self.wo(K.wkv_out(o, self.norm, g, self.eps, padded_rows(b.n_tokens, self.nv, self.wo, r), a.heads, a.dim))
+        return K.linear(self.wo, K.wkv_out(o, self.norm, g, self.eps, padded_rows(b.n_tokens, self.nv, self.wo, r), a.heads, a.dim), b.tickets, slabs=True)
 
     def advance(self, r, k, v, g, z, b: StepBatch, y: Optional[torch.Tensor] = None, index: Optional[int] = None) -> torch.Tensor:
         """the step behind the projections -> the wo projection's input"""
@@ -645,7 +647,7 @@ class TimeMix(nn.Module):
         return K.wkv_step(r, k, v, g, z, self.w2, self.w0, self.u, self.norm, self.eps, b.pos, b.slot, b.cache.states[self.owner(index), "wkv"], y)
 
     def step(self, x: torch.Tensor, norm_w: torch.Tensor, b: StepBatch, index: Optional[int] = None) -> torch.Tensor:
-        return self.wo(self.advance(*self._project(x, norm_w, b, None, index), b, index=index))
+        return K.linear(self.wo, self.advance(*self._project(x, norm_w, b, None, index), b, index=index), b.tickets, slabs=True)
 
     def linears(self):
         return [self.proj, self.wo]
@@ -681,8 +683,8 @@ class GatedMLP(nn.Module):
             out.update({"gate.b": (ff,), "up.b": (ff,), "down.b": (d,)})
         return out
 
-    def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return self.down(K.gated_act(self.gate_up(h), self.fp, self.fp, self.a.act, self.gate_up_bias))
+    def forward(self, h: torch.Tensor, tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
+        return K.linear(self.down, K.gated_linear(self.gate_up, h, self.a.act, self.gate_up_bias, tickets), tickets, slabs=True)
 
     def linears(self):
         return [self.gate_up, self.down]
@@ -715,8 +717,8 @@ class PlainMLP(nn.Module):
             out.update({"up.b": (ff,), "down.b": (d,)})
         return out
 
-    def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return self.down(K.gated_act(self.up(h), self.fp, 0, self.a.act, self.up_bias))
+    def forward(self, h: torch.Tensor, tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
+        return K.linear(self.down, K.linear(self.up, h, tickets, act=self.a.act, bias=self.up_bias), tickets, slabs=True)
 
     def linears(self):
         return [self.up, self.down]
@@ -878,14 +880,17 @@ class LayeredTransformer(nn.Module):
         """embedding -> layers -> logits of the rows `want` (None: every row) of the batch b; mixer(layer's mixer, its inputs, index) = its
         pass over the normed input, or (mixers that say so) over the residual and the norm's weight"""
         cfg, w = self.config, self.tok_embeddings.weight
-        norm = dict(eps=cfg.norm_eps, norm_offset=cfg.design.norm_offset)
+        norm = dict(eps=cfg.norm_eps, norm_offset=cfg.design.norm_offset, dtype=w.dtype)
         x = torch.empty(b.tokens.numel(), cfg.dim, device=w.device, dtype=torch.float32)
 
         def entry(i):
             """what the residual kernel leaves for layer i: its normed input, or nothing"""
             return dict(pre_w=None if self.layers[i].mix.from_residual else self.layers[i].norm1)
 
-        h = K.resid_norm(x, tokens=b.tokens, embed=w, **entry(0), **norm)
+        # a few rows: the products are teal_rows_gemm's, which need a set of counters that no other pass uses at the same time
+        rows = min(x.shape[0], n_want or x.shape[0])
+        b.tickets = torch.empty(K.TICKETS, device=w.device, dtype=torch.int32) if w.dtype != torch.float32 and rows <= K.ROWS_MAX else None
+        h = K.resid_norm(x, tokens=b.tokens, embed=w, **entry(0), **norm, zero=b.tickets)
         for i, layer in enumerate(self.layers):
             last = i + 1 == len(self.layers)
             after = dict(pre_w=self.norm if n_want else None) if last else entry(i + 1)
@@ -895,14 +900,14 @@ class LayeredTransformer(nn.Module):
             y = mixer(layer.mix, (x, layer.norm1) if layer.mix.from_residual else (h,), i)
             h = K.resid_norm(x, y=y, post_w=layer.norm1b, **first, **norm)
             if layer.mlp is not None:
-                h = K.resid_norm(x, y=layer.mlp(h), y_bias=layer.mlp.down_bias, post_w=layer.norm2b, **after, **norm)
+                h = K.resid_norm(x, y=layer.mlp(h, b.tickets), y_bias=layer.mlp.down_bias, post_w=layer.norm2b, **after, **norm)
             if hook is not None:
                 hook(i, x)
         if not n_want:
             return None
         if hook is not None and want is not None:
             h = h[want.long()]
-        return K.softcap(self.output(h), cfg.vocab_size, cfg.logit_softcap)
+        return K.head(self.output, h, cfg.vocab_size, cfg.logit_softcap, b.tickets)
 
     @torch.no_grad()
     def prompt_pass(self, b: PromptBatch, want, hook=None) -> Optional[torch.Tensor]:

@@ -4,6 +4,7 @@ teal_latent_*, teal_grouped_*, teal_wkv_*): shape checks, dtype codes and the la
 Activations and weights fp16, bf16 or true fp32; there is no CPU path."""
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -36,15 +37,102 @@ def _rows(t: torch.Tensor) -> int:
     return t.stride(0)
 
 
-def resid_norm(x, *, tokens=None, embed=None, y=None, y_bias=None, post_w=None, pre_w=None, eps=1e-6, rows=None, dtype=None, norm_offset=0.0):
+class RowsGemm(ctypes.Structure):  # teal_rows_gemm_t
+    _fields_ = [(n, ctypes.c_void_p) for n in ("x", "w", "w_up", "bias", "bias_up", "y", "part")] + [("part_bytes", ctypes.c_size_t), ("tickets", ctypes.c_void_p)] + \
+        [(n, ctypes.c_int) for n in ("M", "K", "N", "ldx", "ld", "ldy", "mode", "act", "n_valid")] + [("softcap", ctypes.c_float)]
+
+
+ROWS_MAX, ROWS_PAIR_MAX = 64, 32  # rows of teal_rows_gemm; of its gate | up form: past them the vendor's product and gated_act are faster (64 rows, 4096 ->
+# 2 x 11008: 55 us against 44 + 6; 32 rows: 38 us against 38 + 6)
+ROWS_ROUNDED, ROWS_SLABS, ROWS_F32 = 0, 1, 2
+TICKETS = 256
+
+
+def rows_weight(lin) -> Optional[torch.Tensor]:
+    """the weight of a plain linear whose product may bypass the module, else None (hooks, another class, a bias)"""
+    if type(lin) is not torch.nn.Linear or lin.bias is not None or lin._forward_hooks or lin._forward_pre_hooks:
+        return None
+    return lin.weight
+
+
+def rows_split(x, w, paired: bool = False) -> int:
+    """slices teal_rows_gemm takes for x [M, K] and the column-major w [N, K]; 0: not a case for it"""
+    M, (N, Kd) = x.shape[0], w.shape
+    if paired:
+        N //= 2
+    if (M > (ROWS_PAIR_MAX if paired else ROWS_MAX) or w.dtype not in (torch.float16, torch.bfloat16) or x.dtype != w.dtype or not w.is_cuda or w.stride(0) != 1
+            or w.stride(1) < w.shape[0] or w.stride(1) & 7 or x.stride(1) != 1 or x.stride(0) & 7 or (w.data_ptr() | x.data_ptr()) & 15):
+        return 0
+    if (N & 7) or Kd * w.stride(1) * 2 > 0xFFF00000:
+        return 0
+    return int(_lib.load().teal_rows_split(M, Kd, N, int(paired)))
+
+
+def _rows_gemm(x, w, N, split, mode, tickets, y, w_up=None, bias=None, bias_up=None, act=-1, n_valid=0, softcap=0.0):
+    tile = 64 if w_up is not None else 128
+    part = None
+    if split > 1 and mode != ROWS_SLABS:
+        part = torch.empty(split * x.shape[0] * (-(-N // tile) * 128), device=x.device, dtype=torch.float32)
+    a = RowsGemm(x=x.data_ptr(), w=w.data_ptr(), w_up=w_up, bias=_p(bias), bias_up=_p(bias_up), y=y.data_ptr(), part=_p(part), part_bytes=0 if part is None else part.numel() * 4,
+                 tickets=_p(tickets), M=x.shape[0], K=w.shape[1], N=N, ldx=x.stride(0), ld=w.stride(1), ldy=y.stride(-2), mode=mode, act=act, n_valid=n_valid, softcap=softcap)
+    _run("teal_rows_gemm", ctypes.byref(a), runtime.dtype_code(x.dtype))
+    return y
+
+
+def linear(lin, x, tickets=None, slabs: bool = False, weight=None, act: Optional[str] = None, bias=None):
+    """act(x W^T + bias) of a linear (or of rows of its weight).  With `tickets` (zero counters, left zero: one set per pass) a few rows go through
+    teal_rows_gemm; `slabs`: the result may then be the product's fp32 partial sums [slices, rows, columns] instead, for resid_norm to add"""
+    w = (rows_weight(lin) if tickets is not None else None) if weight is None else weight
+    split = rows_split(x, w) if w is not None and tickets is not None else 0
+    if split == 0:
+        y = lin(x) if weight is None else torch.nn.functional.linear(x, weight)
+        return y if act is None else gated_act(y, y.shape[1], 0, act, bias)
+    M, N = x.shape[0], w.shape[0]
+    if slabs and act is None:
+        return _rows_gemm(x, w, N, split, ROWS_SLABS, None, torch.empty(split, M, N, device=x.device, dtype=torch.float32))
+    return _rows_gemm(x, w, N, split, ROWS_ROUNDED, tickets, torch.empty(M, N, device=x.device, dtype=x.dtype), bias=bias, act=-1 if act is None else ACTS[act])
+
+
+def gated_linear(lin, x, act: str, bias=None, tickets=None):
+    """act(gate + bias) * (up + bias) of a linear whose output is [gate | up]"""
+    w = rows_weight(lin) if tickets is not None else None
+    N = lin.out_features // 2
+    split = rows_split(x, w, True) if w is not None and not N & 63 else 0
+    if split == 0:
+        return gated_act(lin(x), N, N, act, bias)
+    y = torch.empty(x.shape[0], N, device=x.device, dtype=x.dtype)
+    return _rows_gemm(x, w, N, split, ROWS_ROUNDED, tickets, y, w_up=w.data_ptr() + 2 * N, bias=None if bias is None else bias[:N], bias_up=None if bias is None else bias[N:],
+                      act=ACTS[act])
+
+
+def head(lin, h, vocab: int, cap: Optional[float], tickets=None):
+    """fp32 logits [rows, vocab], soft-capped"""
+    w = rows_weight(lin) if tickets is not None else None
+    split = rows_split(h, w) if w is not None else 0
+    if split == 0:
+        return softcap(lin(h), vocab, cap)
+    out = torch.empty(h.shape[0], vocab, device=h.device, dtype=torch.float32)
+    return _rows_gemm(h, w, w.shape[0], split, ROWS_F32, tickets, out, n_valid=vocab, softcap=float(cap or 0.0))
+
+
+def resid_norm(x, *, tokens=None, embed=None, y=None, y_bias=None, post_w=None, pre_w=None, eps=1e-6, rows=None, dtype=None, norm_offset=0.0, zero=None):
     """x (fp32 [T, D], in place) = embedding rows | x, + [post norm](y + bias); returns h = RMSNorm(x) * (norm_offset + pre_w) (rows of
-    `rows`, packed)"""
+    `rows`, packed).  y: 16-bit, or slabs of `linear`; zero: counters to clear on the way"""
     assert x.dtype == torch.float32 and x.is_contiguous()
     n = x.shape[0] if rows is None else rows.numel()
+    slabs = y is not None and y.dim() == 3
     dtype = dtype or (pre_w if pre_w is not None else embed if embed is not None else y).dtype
     h = torch.empty(n, x.shape[1], device=x.device, dtype=dtype) if pre_w is not None else None
-    _run("teal_layer_resid_norm", _p(x), n, x.shape[1], _p(tokens), _p(embed), 0 if embed is None else embed.shape[0], _p(y),
-         0 if y is None else _rows(y), _p(y_bias), _p(post_w), _p(pre_w), float(norm_offset), float(eps), _p(h), _p(rows), dtype_code(dtype))
+    head = (_p(x), n, x.shape[1], _p(tokens), _p(embed), 0 if embed is None else embed.shape[0], _p(y))
+    tail = (_p(y_bias), _p(post_w), _p(pre_w), float(norm_offset), float(eps), _p(h), _p(rows))
+    if slabs:
+        assert y.dtype == torch.float32 and y.is_contiguous()
+        _run("teal_layer_resid_norm_slabs", *head, y.shape[0], y.shape[1], y.shape[2], *tail, _p(zero), 0 if zero is None else zero.numel(), dtype_code(dtype))
+    elif zero is not None:
+        assert y is None
+        _run("teal_layer_resid_norm_slabs", *head, 0, 0, 0, *tail, _p(zero), zero.numel(), dtype_code(dtype))
+    else:
+        _run("teal_layer_resid_norm", *head, 0 if y is None else _rows(y), *tail, dtype_code(dtype))
     return h
 
 

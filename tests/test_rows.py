@@ -63,3 +63,87 @@ def test_prompt_gemm_producers(Z, n0, n1, T, dtype):
         assert rc == 0 and 1 <= split.value <= 16
         got = slabs[: split.value * N * R].view(split.value, N, R).sum(0)[:, :T].T
         _close(got, x[:, :T].T.float(), w.float(), dtype, steps)
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("M,K,N", [(1, 32, 8), (2, 96, 72), (16, 4096, 4096), (17, 288, 136), (32, 1056, 264), (33, 4096, 200), (64, 11008, 384), (5, 16384, 64)])
+def test_rows_gemm(M, K, N, dtype):
+    """every output of teal_rows_gemm: part tiles of rows and columns, one slice and several (fewer steps than waves, unequal slices), rows of x
+    and y further apart than their columns; slabs and complete sums agree bit for bit; the counters come back zero"""
+    from teal_amd import _lib, runtime
+    from teal_amd.kernels import layered as Kn
+    runtime.init()
+    dt = DT[dtype]
+    g = torch.Generator(device=DEV).manual_seed(K + M)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    img = _image(K, 2 * N, dtype, 3)
+    w, wu = img[:, :N].T, img[:, N:2 * N].T
+    x = torch.full((M, K + 24), float("nan"), device=DEV, dtype=dt)[:, :K]
+    x.copy_(r(M, K).to(dt))
+    bias, bias_up = r(N).to(dt), r(N).to(dt)
+    tickets = torch.zeros(Kn.TICKETS, device=DEV, dtype=torch.int32)
+    split = Kn.rows_split(x, w)
+    assert split == _lib.load().teal_rows_split(M, K, N, 0) >= 1
+    slabs = Kn._rows_gemm(x, w, N, split, Kn.ROWS_SLABS, None, torch.full((split, M, N), float("nan"), device=DEV))
+    _close(slabs.sum(0), x.float(), w.T.float(), dtype)
+    total = slabs[0].clone()
+    for k in range(1, split):
+        total += slabs[k]
+    logits = torch.full((M, N + 3), float("nan"), device=DEV)
+    Kn._rows_gemm(x, w, N, split, Kn.ROWS_F32, tickets, logits, n_valid=N - 3)
+    assert torch.equal(logits[:, : N - 3], total[:, : N - 3]) and bool(torch.isnan(logits[:, N - 3:]).all())
+    out = torch.full((M, N + 4), float("nan"), device=DEV, dtype=dt)
+    for _ in range(3):
+        Kn._rows_gemm(x, w, N, split, Kn.ROWS_ROUNDED, tickets, out)
+        assert torch.equal(out[:, :N], total.to(dt)) and bool(torch.isnan(out[:, N:]).all())
+    step = 2.0 ** (-10 if dtype == 0 else -7)
+    act = Kn.linear(None, x, tickets, weight=w, act="relu2", bias=bias)
+    want = torch.relu(total + bias.float()).square()
+    assert bool(((act.float() - want).abs() <= step * want + 1e-6).all())
+    if N % 64 == 0 and M <= Kn.ROWS_PAIR_MAX:
+        lin = torch.nn.Linear(1, 1, bias=False, device=DEV)
+        lin.weight, lin.out_features = torch.nn.Parameter(img[:, : 2 * N].T, requires_grad=False), 2 * N
+        both = torch.cat([bias, bias_up])
+        got = Kn.gated_linear(lin, x, "gelu_tanh", both, tickets)
+        z, u = (x.double() @ w.T.double() + bias.double()), x.double() @ wu.T.double() + bias_up.double()
+        want = torch.nn.functional.gelu(z, approximate="tanh") * u
+        size = x.double().abs() @ w.T.double().abs()
+        # (the sums' own bound goes through a slope of at most 1.13 and the other factor)
+        assert bool(((got.double() - want).abs() <= step * want.abs() + 2.0 ** -17 * size * (1 + z.abs() + u.abs()) + 1e-6).all())
+        calls = []
+        lin.register_forward_pre_hook(lambda m, a: calls.append(1))  # a hooked module is called, not passed by
+        again = Kn.gated_linear(lin, x, "gelu_tanh", both, tickets)
+        assert calls and bool(((again.double() - want).abs() <= 4 * step * (want.abs() + z.abs() + u.abs() + z.abs() * u.abs())).all())
+    torch.cuda.synchronize()
+    assert not tickets.any()
+
+
+def test_rows_gemm_refuses():
+    from teal_amd.kernels import layered as Kn
+    w = torch.zeros(256, 128 + 8, device=DEV, dtype=torch.float16)[:, :128].T
+    x = torch.zeros(4, 256, device=DEV, dtype=torch.float16)
+    assert Kn.rows_split(x, w) >= 1
+    assert Kn.rows_split(x.float(), w) == 0 and Kn.rows_split(x.bfloat16(), w) == 0 and Kn.rows_split(x, w.contiguous()) == 0
+    assert Kn.rows_split(torch.zeros(65, 256, device=DEV, dtype=torch.float16), w) == 0
+    assert Kn.rows_split(torch.zeros(4, 260, device=DEV, dtype=torch.float16)[:, 2:258], w) == 0    # rows not on 16 bytes
+    assert Kn.rows_split(torch.zeros(4, 264, device=DEV, dtype=torch.float16)[:, :248], w[:, :248]) == 0  # K not a multiple of 32
+    # what is refused there still has its product
+    a, b = torch.randn(3, 248, device=DEV).half(), torch.randn(248, 16, device=DEV).half().T
+    assert torch.equal(Kn.linear(None, a, torch.zeros(256, device=DEV, dtype=torch.int32), weight=b), torch.nn.functional.linear(a, b))
+
+
+@pytest.mark.parametrize("D", [64, 1003, 4096])
+def test_resid_norm_adds_slabs(D):
+    """slabs in slab order, rows picked out of them, counters cleared"""
+    from teal_amd.kernels import layered as Kn
+    T, S = 7, 3
+    x, y = torch.randn(T, D, device=DEV), torch.randn(S, T, D, device=DEV)
+    post, pre = (torch.randn(D, device=DEV).to(torch.bfloat16) for _ in range(2))
+    rows = torch.tensor([5, 1], device=DEV, dtype=torch.int32)
+    s = (y[0] + y[1]) + y[2]
+    norm = lambda t: t * torch.rsqrt(t.square().mean(-1, keepdim=True) + 1e-5)  # noqa: E731
+    want = x + norm(s) * post.float()
+    got, zero = x.clone(), torch.full((256,), 7, device=DEV, dtype=torch.int32)
+    h = Kn.resid_norm(got, y=y, post_w=post, pre_w=pre, eps=1e-5, rows=rows, zero=zero)
+    assert torch.allclose(got[rows.long()], want[rows.long()], atol=1e-5, rtol=1e-5) and torch.equal(got[0], x[0]) and not zero.any()
+    assert torch.allclose(h.float(), (norm(want) * pre.float())[rows.long()], atol=1e-2, rtol=2 ** -7)
