@@ -399,6 +399,23 @@ int teal_prefill_resid_norm(const void* emb, const int32_t* tokens, int T, const
 int teal_prefill_attention(const float* qkv_slabs, int split, const void* rope, void* k_cache, void* v_cache, void* yt, int T, int n_head,
                            int n_kv_head, int head_dim, int max_seq, int dtype, void* stream);
 
+/* ---- Llama prompt pass of any length, teal_amd/csrc/teal_prompt.hip ----------------------------------------------------
+ * 16-bit rows [token][feature]; the rounding points are the module path's 16-bit tensors.  Positions and token ids are device int32 or int64
+ * arrays ([T]; the ..64 flags) and are kept inside their tables. */
+
+/* h[t] = (emb[tokens[t]] | h[t]) + (y[t] | round(sum of n_slabs fp32 slabs [n_slabs][T][dim])); x[t] = RMSNorm(h[t]) * w.  emb / y / slabs optional; dim
+ * % 8 == 0, <= 16384; zero: optional, n_zero <= 256 counters set to zero */
+int teal_prompt_norm(const void* emb, int vocab, const void* tokens, int tokens64, void* h, const void* y, const float* slabs, int n_slabs, const void* w,
+                     void* x, int T, int dim, float eps, unsigned* zero, int n_zero, int dtype, void* stream);
+/* qkv [T][ldq] = q | k | v: q rotated in place, k rotated and v into the rows pos[t] of the caches [n_kv_head][max_seq][head_dim] */
+int teal_prompt_rope(void* qkv, int ldq, const void* rope, const void* pos, int pos64, void* k_cache, void* v_cache, int T, int n_head, int n_kv_head,
+                     int head_dim, int max_seq, int dtype, void* stream);
+/* out[t] = softmax(scale * q[t] K^T) V over the cache rows 0 .. pos[t]; head_dim 64 or 128 */
+int teal_prompt_attention(const void* q, int ldq, const void* k_cache, const void* v_cache, const void* pos, int pos64, void* out, int ldo, int T,
+                          int n_head, int n_kv_head, int head_dim, int max_seq, float scale, int dtype, void* stream);
+/* h[i] = round(silu(gate[i])) * up[i], i < n (n % 8 == 0) */
+int teal_silu_mul(const void* gate, const void* up, void* h, size_t n, int dtype, void* stream);
+
 /* ---- matrix products over a few rows, teal_amd/csrc/teal_rows.hip -----------------------------------------------------
  * y[M][N] = x[M][K] * W^T image [K][ld] for M <= 64, K % 32 == 0, N % 8 == 0, 16-bit operands, fp32 sums (over slices of K in slice order:
  * bit-reproducible).  x rows ldx apart (ldx % 8 == 0), ld % 8 == 0; x, images and biases 16-byte aligned. */

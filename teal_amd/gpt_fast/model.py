@@ -262,6 +262,7 @@ class Transformer(nn.Module):
     # (gpt-fast/generate.py:420 torch.compile(decode_one_token)).  There is no tracing compiler here: a single-token
     # call on a fully patched model runs the hand-fused HIP decode step instead (teal_amd/gpt_fast/engine.py: five
     # launches per layer, same thresholds, same weights, same KV caches, same attribute bundle on the modules).
+    # More than one token: the fused prompt pass (prefill.PromptPass), where it computes what the modules would.
     # `fused_decode = False` keeps the op-by-op module path (tests compare the two).
     fused_decode: bool = True
 
@@ -311,6 +312,12 @@ class Transformer(nn.Module):
             if eng is not None:
                 # a fresh tensor like the op-by-op path returns (the engine's logits buffer is overwritten by the next step)
                 return eng(idx.view(1, 1).to(torch.int32), input_pos.view(1).to(torch.int32)).clone()
+        if (self.fused_decode and idx.numel() > 1 and idx.is_cuda and idx.dim() == 2 and idx.shape[0] == 1 and input_pos is not None and input_pos.is_cuda
+                and input_pos.shape == idx.shape[1:] and idx.dtype in (torch.int32, torch.int64) and input_pos.dtype in (torch.int32, torch.int64)
+                and type(idx) is Tensor and type(input_pos) is Tensor and not torch.is_grad_enabled() and not torch.compiler.is_compiling()):
+            from .prefill import PromptPass
+            if PromptPass.supports(self) is None:
+                return PromptPass.run(self, idx, input_pos)
         mask = self.causal_mask[None, None, input_pos]
         freqs_cis = self.freqs_cis[input_pos]
         x = self.tok_embeddings(idx)

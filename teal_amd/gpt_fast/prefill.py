@@ -23,10 +23,13 @@ import ctypes
 from typing import Optional
 
 import torch
+import torch.nn as nn
 
 from .. import _lib, runtime
+from ..kernels import layered as K
+from ..kernels.sparse_gemv import SparseGEMV, SparseQKVGEMV
 from ..monkeypatch import UP_SHIFT_BYTES, to_column_major
-from .model import Transformer
+from .model import KVCache, RMSNorm, Transformer, TransformerBlock, _sparse_attn_forward, _sparse_ffn_forward
 
 MAX_T = 16  # most tokens of a pass; the hand-over layout is [feature][8] for T <= 8 and [feature][16] for 9 <= T <= 16 (buffers sized for 16)
 IN_XT, IN_NORM, IN_SILU_MUL = 0, 1, 2
@@ -165,6 +168,89 @@ class PrefillEngine:
         if rc != 0:
             _lib.check(rc, "teal_dense_gemv (lm_head)")
         return self.logits
+
+
+class PromptPass:
+    """The prompt pass of any length for a patched 16-bit model: what Transformer.forward runs for more than one token (model.fused_decode), in
+    place of some thirty launches per layer of the op-by-op modules.  Per layer: norm -> wqkv -> rotation and cache rows -> attention over the cache ->
+    wo -> norm -> gate | up, silu * up -> down (csrc/teal_prompt.hip; products over up to 64 rows by csrc/teal_rows.hip, larger ones by the vendor
+    library).  Dense, same rounding points, same results: logits [1, T, vocab] of every token.  Holds no state of its own."""
+
+    @staticmethod
+    def supports(model: Transformer) -> Optional[str]:
+        """None if this pass computes what the modules of `model` would, else the reason it may not be used"""
+        cfg = model.config
+        if int(getattr(model, "tp_world", 1)) > 1:
+            return "tensor-parallel models run their all-reduce hooks"
+        if any(m._forward_hooks or m._forward_pre_hooks for m in model.modules() if m is not model):
+            return "a module has forward hooks"
+        dt, dev = model.output.weight.dtype, model.output.weight.device
+        if dt not in (torch.float16, torch.bfloat16) or dev.type != "cuda":
+            return f"weights are {dt} on {dev.type}"
+        if cfg.head_dim not in (64, 128) or cfg.dim != cfg.n_head * cfg.head_dim or cfg.dim > 16384:
+            return "head_dim 64 / 128, dim = n_head * head_dim <= 16384"
+        if model.freqs_cis is None or model.freqs_cis.dtype != dt or model.freqs_cis.shape[0] < model.max_seq_length or not model.freqs_cis.is_contiguous():
+            return "caches are not set up in the model dtype, or hold more positions than the rotation table"
+        if type(model.norm) is not RMSNorm or type(model.tok_embeddings) is not nn.Embedding or model.tok_embeddings.max_norm is not None:
+            return "replaced modules"
+        weights = [model.output, model.tok_embeddings, model.norm]
+        for layer in model.layers:
+            at, ff = layer.attention, layer.feed_forward
+            if type(layer) is not TransformerBlock or "forward" in layer.__dict__ or type(layer.attention_norm) is not RMSNorm or type(layer.ffn_norm) is not RMSNorm:
+                return "replaced modules"
+            for m, fn, g1 in ((at, _sparse_attn_forward, SparseQKVGEMV), (ff, _sparse_ffn_forward, SparseGEMV)):
+                if getattr(m.__dict__.get("forward"), "__func__", None) is not fn or getattr(m, "int4", False) or getattr(m, "int8", False):
+                    return "not a 16-bit patched block"
+                for k, op, cls in ((m.gemv1_kernel, m.gemv1, g1), (m.gemv2_kernel, m.gemv2, SparseGEMV)):
+                    if type(k) is not cls or op is not k.operator(True):
+                        return "replaced operators"
+            kc = at.kv_cache
+            if type(kc) is not KVCache or any(c.dtype != dt or c.shape[0] != 1 or c.shape[2] != model.max_seq_length or not c.is_contiguous() for c in (kc.k_cache, kc.v_cache)):
+                return "KV caches must be contiguous with max_batch_size == 1"
+            weights += [at.wqkv, at.wo, ff.w1, ff.w2, ff.w3, layer.attention_norm, layer.ffn_norm]
+        if any(w.weight.dtype != dt or w.weight.device != dev or getattr(w, "bias", None) is not None for w in weights):
+            return "mixed dtypes or devices, or biases"
+        if any(type(w) is not nn.Linear for w in weights if hasattr(w, "out_features")):
+            return "replaced modules"
+        return None
+
+    @staticmethod
+    def run(model: Transformer, idx: torch.Tensor, input_pos: torch.Tensor) -> torch.Tensor:
+        """idx [1, T], input_pos [T] (any positions of the cache) -> logits [1, T, vocab]; the caller asked `supports`"""
+        m, cfg, L, st = model, model.config, _lib.load(), runtime.stream_ptr()
+        w0 = m.output.weight
+        dt, dev, code, T, D, hd = w0.dtype, w0.device, runtime.dtype_code(w0.dtype), idx.numel(), cfg.dim, cfg.head_dim
+        tokens, pos = idx.reshape(-1).contiguous(), input_pos.contiguous()
+        eps, scale, max_seq, few = float(cfg.norm_eps), hd ** -0.5, m.max_seq_length, T <= K.ROWS_MAX
+        new = lambda *shape: torch.empty(*shape, device=dev, dtype=dt)  # noqa: E731
+        tickets = torch.empty(K.TICKETS, device=dev, dtype=torch.int32) if few else None
+        h, x = new(T, D), new(T, D)
+
+        def norm(w, y=None, emb=None):
+            slabs = y is not None and y.dim() == 3
+            _lib.check(L.teal_prompt_norm(None if emb is None else emb.data_ptr(), 0 if emb is None else emb.shape[0], None if emb is None else tokens.data_ptr(),
+                                          int(tokens.dtype == torch.int64), h.data_ptr(), y.data_ptr() if y is not None and not slabs else None,
+                                          y.data_ptr() if slabs else None, y.shape[0] if slabs else 0, w.data_ptr(), x.data_ptr(), T, D, eps,
+                                          tickets.data_ptr() if emb is not None and few else None, K.TICKETS, code, st), "teal_prompt_norm")
+
+        layers = list(m.layers)
+        norm(layers[0].attention_norm.weight, emb=m.tok_embeddings.weight)
+        for i, layer in enumerate(layers):
+            at, ff = layer.attention, layer.feed_forward
+            kc, vc = at.kv_cache.k_cache.data_ptr(), at.kv_cache.v_cache.data_ptr()
+            qkv, y = K.linear(at.wqkv, x, tickets), new(T, D)
+            _lib.check(L.teal_prompt_rope(qkv.data_ptr(), qkv.stride(0), m.freqs_cis.data_ptr(), pos.data_ptr(), int(pos.dtype == torch.int64), kc, vc, T, cfg.n_head,
+                                          cfg.n_local_heads, hd, max_seq, code, st), "teal_prompt_rope")
+            _lib.check(L.teal_prompt_attention(qkv.data_ptr(), qkv.stride(0), kc, vc, pos.data_ptr(), int(pos.dtype == torch.int64), y.data_ptr(), D, T, cfg.n_head,
+                                               cfg.n_local_heads, hd, max_seq, scale, code, st), "teal_prompt_attention")
+            norm(layer.ffn_norm.weight, K.linear(at.wo, y, tickets, slabs=True))
+            mid = K.gated_pair(ff.w1, ff.w3, x, "silu_rounded", tickets)
+            if mid is None:
+                gate, up = K.linear(ff.w1, x, tickets), K.linear(ff.w3, x, tickets)
+                mid = gate  # (in place)
+                _lib.check(L.teal_silu_mul(gate.data_ptr(), up.data_ptr(), mid.data_ptr(), mid.numel(), code, st), "teal_silu_mul")
+            norm(layers[i + 1].attention_norm.weight if i + 1 < len(layers) else m.norm.weight, K.linear(ff.w2, mid, tickets, slabs=True))
+        return K.linear(m.output, x, tickets).view(1, T, -1)
 
 
 class FusedPrefill:

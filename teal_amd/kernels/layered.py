@@ -12,7 +12,7 @@ import torch
 from .. import _lib, runtime
 
 F32 = 2
-ACTS = {"silu": 0, "gelu_tanh": 1, "relu2": 2}
+ACTS = {"silu": 0, "gelu_tanh": 1, "relu2": 2, "silu_rounded": 3}  # (silu_rounded: gate | up products of teal_rows_gemm only)
 NO_WINDOW = 1 << 30  # a window wider than any sequence: plain causal attention
 TILE = 64            # packed key spans of a prompt pass are padded to this many rows
 
@@ -103,6 +103,17 @@ def gated_linear(lin, x, act: str, bias=None, tickets=None):
     y = torch.empty(x.shape[0], N, device=x.device, dtype=x.dtype)
     return _rows_gemm(x, w, N, split, ROWS_ROUNDED, tickets, y, w_up=w.data_ptr() + 2 * N, bias=None if bias is None else bias[:N], bias_up=None if bias is None else bias[N:],
                       act=ACTS[act])
+
+
+def gated_pair(gate, up, x, act: str, tickets=None):
+    """round(act(gate)) * up of two linears of one shape and layout, or None: not a case for teal_rows_gemm"""
+    w, u = (rows_weight(lin) if tickets is not None else None for lin in (gate, up))
+    if w is None or u is None or w.shape != u.shape or w.stride() != u.stride() or u.data_ptr() & 15 or x.shape[0] > ROWS_PAIR_MAX or w.shape[0] & 63:
+        return None
+    if rows_split(x, w) == 0:
+        return None
+    split = int(_lib.load().teal_rows_split(x.shape[0], w.shape[1], w.shape[0], 1))
+    return _rows_gemm(x, w, w.shape[0], split, ROWS_ROUNDED, tickets, torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype), w_up=u.data_ptr(), act=ACTS[act])
 
 
 def head(lin, h, vocab: int, cap: Optional[float], tickets=None):
