@@ -101,6 +101,7 @@ struct DeviceCtx {
     int num_cu;       // 0: not initialised yet
     bool gqa_lds_ok;  // the grouped-query attention kernel may take kGqaMaxLds of LDS on this device
     bool prefill_lds_ok;  // the prompt-pass GEMM may take kPrefillLds
+    bool int4_lds_ok;     // the int4 GEMV may take kI4MaxLds
     bool rows_lds_ok;     // the products over a few rows may take rows_lds()
 };
 DeviceCtx* device_ctx();                   // context of the CURRENT device (nullptr: no device)
@@ -110,6 +111,7 @@ inline int num_cu_or(int dflt) {           // CU count of the current device, or
 }
 bool attention_device_init();              // teal_attention.hip: per-kernel attributes of the current device
 bool prefill_device_init();                // teal_prefill.hip: alike
+bool int4_device_init();                   // teal_gemv_int4.hip: alike
 bool rows_device_init();                   // teal_rows.hip: alike
 // teal_fused_gemv over int4 group-quantised weights (out->weight_bits == 4): teal_gemv_int4.hip
 int fused_gemv_i4(const teal_gemv_in_t* in, const teal_gemv_out_t* out, int Z, int dtype, void* ws, size_t ws_bytes,

@@ -9,26 +9,30 @@
 //
 // Weight layout (ours to choose — the reference's packed layout is tinygemm's): the image of W^T by ROW PAIRS,
 // wq[Z / 2][ldb] bytes; dword g of pair-row p holds columns 4g .. 4g+3 of row 2p in its low half (nibble j = column 4g+j)
-// and of row 2p+1 in its high half.  One mask-and-or under an fp16 exponent then yields the half2 (1024 + q[2p][c],
-// 1024 + q[2p+1][c]) and one v_dot2_f32_f16 against (x[2p], x[2p+1]) does two multiply-adds in fp32: ~1.2 VALU instructions
-// per multiply-add where a row-per-dword layout needs ~2.6 (unpack, convert, fma) — and this kernel is bound by the VALU,
-// not by HBM: 4 waves per SIMD share it, and at 4 bits a byte of weights carries 4x the arithmetic of fp16.  A pair is
-// fetched when EITHER row is kept (the other row's x enters as 0, which is exact): at 50 % sparsity 75 % of the pairs,
-// i.e. 1.5x the bytes of a row-granular gather — bytes this kernel has to spare.
+// and of row 2p+1 in its high half.  One mask-and-or under a 16-bit exponent yields (1024 + q[2p][c], 1024 + q[2p+1][c])
+// (fp16; bf16: 128 + q), two of the eight inputs of one column that a lane hands the matrix cores.  A pair is
+// fetched when EITHER row is kept (the other row's x enters as 0, which is exact): at 50 % sparsity 75 % of the pairs.
 //
-// Kernel: one 16-wave workgroup = one 128-column tile x one slice of the 32-row units.  A wave owns units; per unit it
-// ballots the keep mask, compacts the kept pairs into its LDS lists, deals them to its four 16-lane groups (a lane = 8
-// columns = 8 bytes of a 128-byte pair-row segment), accumulates A = sum x * (bias + q) and X = sum x in fp32 and applies
-// scale / zero ONCE per (unit, column):  y += scale * (A - (bias + 8) X) + zero * X  — the group parameters cost 32 bytes
-// per lane and unit instead of per row.  Split-K over units is folded into the one launch by arrival tickets (the last
-// slice of a tile sums the partials in slice order: deterministic, no atomics on the data).  No MFMA on purpose.
+// Kernel: one 16-wave workgroup = one 128-column tile x one slice of the 32-row units; a wave takes every sixteenth unit.  The
+// workgroup leaves its slice's activations masked in LDS; a lane (8 columns, the four pairs of its 16-lane group) reads its eight
+// with one LDS read, requests the pairs whose activations are not both zero (the others at an offset outside the buffer
+// resource: no traffic, no list, no branch), and eight MFMAs give sum x * (bias + q) of the unit's 32 rows, a ninth, over ones,
+// X = sum x.  Scale and zero are applied ONCE per (unit, column):  y += scale * (A - (bias + 8) X) + zero * X.  The 16 waves keep
+// one unit each in flight.  Split-K over units is folded into the one launch by arrival tickets (the last slice of a tile sums the
+// partials in slice order: deterministic, no atomics on the data).
+//
+// What bounds it: the vector ALU (72 instructions per unit and wave, half of them nibbles becoming halves), then the launch's fixed 4 - 5
+// us; the stream (weights and, at G = 32, a quarter as many bytes of group parameters) hides behind them: with nothing kept a launch is
+// only a fifth faster.  Llama-2-7B at G = 32 and 50 %: gate|up 16.8 -> 15.1, qkv 11.7 -> 10.5, down 8.6 -> 7.5, wo 7.8 -> 5.7 us.
+// The kernel before this one compacted the kept pairs into lists and walked them with v_dot2, 16 dot products and 9 list
+// instructions per pair and lane: bound by the vector ALU and by its passes (ballots -> lists -> loads -> products, nothing of one
+// pass in flight during the next).
 //
 // The kernel takes the producers of the fused decode step like the 16-bit one (teal_gemv_fast.h): MODE 1 residual + fp32
-// slabs -> RMSNorm (every workgroup recomputes the vector into LDS: the norm needs all of it), MODE 2 silu(gate) * up and
-// MODE 4 split-KV attention merge (element-wise: each wave builds the 32 activations of its own units in registers) — and
-// leaves either rounded outputs or its fp32 split-K partials as slabs for the next launch's producer, so an int4 layer is
-// 5 launches too.
-#include "teal_common.h"
+// slabs -> RMSNorm (every workgroup recomputes the whole vector: the norm needs all of it), MODE 2 silu(gate) * up and
+// MODE 4 split-KV attention merge (element-wise: a workgroup builds its own slice) — and leaves either rounded outputs or its
+// fp32 split-K partials as slabs for the next launch's producer, so an int4 layer is 5 launches too.
+#include "teal_rows_core.h"
 
 #include <limits.h>
 
@@ -40,12 +44,10 @@
 
 namespace teal {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 constexpr int kPhaseRow = 32;  // uint64 stamps per workgroup (as in teal_gemv_kernel.h)
 
 struct I4Seg {
-    const unsigned char* wq;  // first byte of the segment's columns in row 0
+    const unsigned char* wq;  // first byte of the segment's columns in pair-row 0
     const uint16_t* sz;       // (scale, zero) of the segment's first column in group 0
     uint16_t* y;              // rounded output of the segment (null when the launch leaves slabs)
     int ldb, szld;            // pair-row stride of wq in bytes; columns per row of sz
@@ -73,55 +75,29 @@ struct I4Args {
     unsigned long long* phase;  // PHASE instantiations: kPhaseRow stamps per workgroup (teal_set_phase_buffer)
 };
 
-// A wave handles its 32-row units in PASSES of four: the activations of the pass first; the ballots compact the kept row
-// PAIRS of each unit into the wave's LDS lists (pair index, and the two activations as a half2 with a dropped row's at 0)
-// with mbcnt ranks; then each of the wave's four 16-lane groups takes ONE unit of the pass — its own group parameters, its
-// own accumulators, no cross-lane traffic until the end of the kernel — and EVERY pair-row load of the pass is issued before
-// the first is consumed.  (Four groups sharing the pairs of one unit would each fetch that unit's 32 bytes of parameters
-// per lane: the launch was then bound by the CU's 64 bytes / clock of vector-memory issue, half of it those parameters.)
-// scale / zero are applied per UNIT with the parameters of the unit's group — y += scale * (A_u - c X_u) + zero * X_u is
-// linear in the units of a group — so units are independent whatever the group size.  fp16 activations: nibbles 1 and 3 of
-// a half are used where they lie, as 1024 + 16 q (no shift); their columns are rescaled at the flush.  bf16 activations:
-// bias 128 (7 mantissa bits), every nibble shifted down.
-// PHASE (measurement builds only): thread 0 stamps [0] entry, [1] arguments in registers, [2] producer done (MODE 1), and for
-// its wave's first pass [3] activations ready, [4] list written, [5] every load issued, [6] first unit consumed, [7] pass
-// done; [8] all passes done, [9] past the reduce barrier, [10] outputs stored.  100 MHz wall clock (scripts/int4_phase.py).
-// KIND, by the units a launch leaves a wave (host: fused_gemv_i4):
-//   1 SHARE  one or two (the 7B wo projection over 256 workgroups: one) — the four lane groups SHARE each unit, pairs dealt
-//            round-robin, instead of three of them idling while one walks 12 pairs on its own;
-//   0 GROUP  more: passes of four units, one unit per lane group, loads issued only for the pairs that exist.
-// (A software-pipelined form of GROUP — pass p + 1's loads in flight while pass p is consumed, every lane issuing exactly 16
-// loads and running 16 steps per pass so that the loop body is straight-line and the compiler's vmcnt waits exact — measured
-// SLOWER: 494 against 537 tok/s on Llama-2-7B, 66.4 against 89.1 on Llama-2-70B, int4-g32 @ 50 %; 128 VGPRs with spills,
-// 17 % more loads and steps than the pairs that exist.  Starting the odd waves half a pass late, so that one half of the
-// chip's waves loads while the other computes: 88.1 / 86.2 against 89.4 tok/s (70B), 533 / 523 against 539 (7B).  A ring of 8
-// loads per lane that never drains between passes, the next pass's lists built while the current one streams (ISA checked:
-// exact progressive vmcnt waits): 561 against 578, 97.4 against 102.9.  Passes of eight units, two per lane group (32 loads in
-// flight per lane, the 7B gate|up launch in one pass): 567 against 578, 99.4 against 102.8.  None is kept: overlap inside a wave is not what
-// bounds the launch — padding every unit to 16 steps costs more than the overlap returns.)
-constexpr int kI4Group = 0, kI4Share = 1;
-template <bool BF16, int MODE, int KIND, bool PHASE = false>
+// fp16 activations: nibbles 1 and 3 of a half are used where they lie, as 1024 + 16 q (no shift); their columns are rescaled when
+// scale and zero are applied.  bf16 activations: bias 128 (7 mantissa bits), every nibble shifted down.
+// PHASE (measurement builds only): thread 0 stamps [0] entry, [1] arguments in registers, [2] MODE 1's producer done, [3] activations in LDS,
+// [5] first unit requested, [6] first unit consumed, [8] all units done, [9] past the reduce barrier, [10] outputs stored.
+// 100 MHz wall clock (scripts/int4_phase.py).
+constexpr size_t kI4MaxLds = 128 * 1024 + 64;  // masked activations of a slice (65536 rows) and one unit of zeros
+template <bool BF16, int MODE, bool PHASE = false>
 __global__ __launch_bounds__(1024) void sparse_gemv_int4_kernel(const I4Args a) {
-    constexpr bool SHARE = KIND == kI4Share;
-    constexpr int WAVES = 16, BN = 128, UP = SHARE ? 2 : 4;  // UP: units per pass
+    constexpr int WAVES = 16, BN = 128, DEPTH = 1;  // DEPTH: units of a wave in flight (2, 3, 4: 4, 7, 11 % slower per token)
     unsigned long long t_entry = 0;
     if constexpr (PHASE) t_entry = wall_clock64();
-    extern __shared__ __align__(16) uint16_t xs[];  // MODE 1: the normalised activation vector, Z entries
-    __shared__ float red[WAVES * BN];
-    // 16 slots per unit: ascending; SHARE: rank k at slot (k & 3) * 4 + (k >> 2), a lane group's four entries contiguous
-    __shared__ __align__(16) uint8_t list_i[WAVES][UP * 16];   // pair index inside the unit (one byte: a lane's 16 in one read)
-    __shared__ __align__(16) uint32_t list_x[WAVES][UP * 16];  // (x[2p], x[2p + 1]) as 16-bit halves, a dropped row's = 0
+    extern __shared__ __align__(16) uint16_t xs[];  // masked activations: MODE 1 the whole vector, else the slice's units back to back
+    __shared__ __align__(16) float red[WAVES * BN];
     __shared__ float wsum[WAVES];
     __shared__ float tflag;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = blockIdx.x, slice = blockIdx.y, split = gridDim.y;
-    const int rs = lane >> 4, cl = lane & 15;  // pair slot of the wave, 8-byte column slot of the tile
+    const int g = lane >> 4, cl = lane & 15;  // the lane's four pairs of a unit, its 8 columns of the tile
     const int Z = a.Z;
-    bool first_pass = true;
     auto stamp = [&](const int i) {
         if constexpr (PHASE) {
-            if (a.phase && tid == 0 && first_pass) a.phase[(size_t)(blockIdx.y * gridDim.x + blockIdx.x) * kPhaseRow + i] = wall_clock64();
+            if (a.phase && tid == 0) a.phase[(size_t)(blockIdx.y * gridDim.x + blockIdx.x) * kPhaseRow + i] = wall_clock64();
         }
     };
     // ONE batch of scalar loads for every kernel argument, up front (an "s" input forces the value into an SGPR here):
@@ -138,6 +114,25 @@ __global__ __launch_bounds__(1024) void sparse_gemv_int4_kernel(const I4Args a) 
     }
     stamp(1);
 
+    // ---- this workgroup's column tile: segment, threshold, weight image ---------------------------------------------------
+    // (selected field by field from kernel arguments already in SGPRs: indexing a.seg[] by a run-time s would be a
+    // dependent scalar load)
+    int s = 0;
+    if (a.nseg > 1 && tile >= a.seg[1].tile0) s = 1;
+    if (a.nseg > 2 && tile >= a.seg[2].tile0) s = 2;
+#define TEAL_I4_SEG(f) (s == 0 ? a.seg[0].f : (s == 1 ? a.seg[1].f : a.seg[2].f))
+    const unsigned char* seg_wq = TEAL_I4_SEG(wq);
+    const uint16_t* seg_sz = TEAL_I4_SEG(sz);
+    uint16_t* seg_y = TEAL_I4_SEG(y);
+    const int ldb = TEAL_I4_SEG(ldb), szld = TEAL_I4_SEG(szld), seg_tile0 = TEAL_I4_SEG(tile0);
+    const float tau = TEAL_I4_SEG(tau);
+#undef TEAL_I4_SEG
+    auto masked = [&](const uint32_t b) -> uint16_t {
+        const float v = bits_to_float(b, BF16);
+        return keep_rule(v, tau) || v != v ? (uint16_t)b : (uint16_t)0;
+    };
+    // unit u belongs to slice u % split, and inside the slice, as its k-th, to wave k % 16
+    const int nunits = Z >> 5, nk = (nunits - slice + split - 1) / split;
     // ---- producer -------------------------------------------------------------------------------------------------------
     if constexpr (MODE == 1) {
         // h = resid + round(sum slabs);  x = round(round(h * rstd) * w)          gpt-fast/model.py:158-161, 289-291
@@ -198,7 +193,7 @@ __global__ __launch_bounds__(1024) void sparse_gemv_int4_kernel(const I4Args a) 
                 if (m < Z) {
                     const uint32_t hb = xs[m];  // this thread's own element
                     const float xn = bits_to_float(float_to_bits<BF16>(bits_to_float(hb, BF16) * rstd), BF16);
-                    xs[m] = float_to_bits<BF16>(xn * bits_to_float(wb[k], BF16));
+                    xs[m] = masked(float_to_bits<BF16>(xn * bits_to_float(wb[k], BF16)));
                     if (writer) a.resid_out[m] = (uint16_t)hb;
                 }
             }
@@ -206,286 +201,175 @@ __global__ __launch_bounds__(1024) void sparse_gemv_int4_kernel(const I4Args a) 
         if (Z <= 4096) produce(std::integral_constant<int, 4>{});
         else if (Z <= 8192) produce(std::integral_constant<int, 8>{});
         else produce(std::integral_constant<int, 16>{});
+        if (tid < 32) xs[Z + tid] = 0;
         __syncthreads();
     }
 
     stamp(2);
-    // ---- this workgroup's column tile: segment, threshold, weight image ---------------------------------------------------
-    // (selected field by field from kernel arguments already in SGPRs: indexing a.seg[] by a run-time s would be a
-    // dependent scalar load)
-    int s = 0;
-    if (a.nseg > 1 && tile >= a.seg[1].tile0) s = 1;
-    if (a.nseg > 2 && tile >= a.seg[2].tile0) s = 2;
-#define TEAL_I4_SEG(f) (s == 0 ? a.seg[0].f : (s == 1 ? a.seg[1].f : a.seg[2].f))
-    const unsigned char* seg_wq = TEAL_I4_SEG(wq);
-    const uint16_t* seg_sz = TEAL_I4_SEG(sz);
-    uint16_t* seg_y = TEAL_I4_SEG(y);
-    const int ldb = TEAL_I4_SEG(ldb), szld = TEAL_I4_SEG(szld), seg_tile0 = TEAL_I4_SEG(tile0);
-    const float tau = TEAL_I4_SEG(tau);
-#undef TEAL_I4_SEG
-    const uint32_t scol = (uint32_t)(tile - seg_tile0) * BN + cl * 8;  // the lane's first column inside the segment
-    // a pair-row holds one byte per column.  Addresses = workgroup-uniform base (scalar registers) + a 32-bit lane offset:
-    // one VGPR and one multiply-add per load instead of a 64-bit pointer each (the host bounds the image below 4 GB)
-    const unsigned char* wtile = seg_wq + (uint32_t)(tile - seg_tile0) * BN;
-    const uint32_t lane_off = (uint32_t)cl * 8u;
-    const uint32_t uldb = (uint32_t)ldb;
-    const uint16_t* szb = seg_sz + (size_t)scol * 2;
-    const int nunits = Z >> 5;
-    uint8_t* li = list_i[wave];
-    uint32_t* lx = list_x[wave];
-    constexpr uint32_t kBias = BF16 ? 0x43004300u : 0x64006400u;  // half2 (128, 128) bf16 / (1024, 1024) fp16
-    constexpr uint32_t kOnes = BF16 ? 0x3F803F80u : 0x3C003C00u;  // half2 (1, 1)
-    auto dot2 = [](const uint32_t w2, const uint32_t x2, const float acc) {
-        if constexpr (BF16) return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w2), __builtin_bit_cast(bf16x2_t, x2), acc, false);
-        else return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, w2), __builtin_bit_cast(f16x2, x2), acc, false);
-    };
-    float total[8];
+    // the element-wise producers: the slice's elements, every load of a round first
+    if constexpr (MODE != 1) {
+        constexpr int R = MODE == 4 ? 2 : 4;
+        const int total = nk * 32;
+        for (int e0 = tid; e0 < total; e0 += 1024 * R) {
+            uint32_t m_el[R], xb[R];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) total[k] = 0.0f;
-    // 16 multiply-adds of a lane: 8 columns x the two rows of a pair
-    auto mac16 = [&](const u32x2 dd, const uint32_t x2, float (&A)[8], float& X) {
+            for (int i = 0; i < R; ++i) {
+                const int e = min(e0 + 1024 * i, total - 1);
+                m_el[i] = ((uint32_t)(slice + split * (e >> 5)) << 5) + (uint32_t)(e & 31);
+            }
+            if constexpr (MODE == 0) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t w = dd[h];
-            if constexpr (BF16) {
+                for (int i = 0; i < R; ++i) xb[i] = a.x[m_el[i]];
+            } else if constexpr (MODE == 2) {
+                // x = round(round(silu(gate)) * up)                                  gpt-fast/model.py:258-259
+                uint32_t gb[R], ub[R];
 #pragma unroll
-                for (int jj = 0; jj < 4; ++jj) A[4 * h + jj] = dot2(((w >> (4 * jj)) & 0x000F000Fu) | kBias, x2, A[4 * h + jj]);
+                for (int i = 0; i < R; ++i) {
+                    gb[i] = a.x[m_el[i]];
+                    ub[i] = a.x[(uint32_t)Z + m_el[i]];
+                }
+#pragma unroll
+                for (int i = 0; i < R; ++i) {
+                    const float gt = bits_to_float(gb[i], BF16);
+                    const float sl = bits_to_float(float_to_bits<BF16>(gt / (1.0f + expf(-gt))), BF16);
+                    xb[i] = float_to_bits<BF16>(sl * bits_to_float(ub[i], BF16));
+                }
             } else {
-                const uint32_t w8 = w >> 8;
-                A[4 * h + 0] = dot2((w & 0x000F000Fu) | kBias, x2, A[4 * h + 0]);
-                A[4 * h + 1] = dot2((w & 0x00F000F0u) | kBias, x2, A[4 * h + 1]);  // 1024 + 16 q
-                A[4 * h + 2] = dot2((w8 & 0x000F000Fu) | kBias, x2, A[4 * h + 2]);
-                A[4 * h + 3] = dot2((w8 & 0x00F000F0u) | kBias, x2, A[4 * h + 3]);  // 1024 + 16 q
-            }
-        }
-        X = dot2(kOnes, x2, X);
-    };
-    // scale / zero of one unit: sum x (q - 8) from the biased accumulators; a dead unit has X = A = 0
-    auto flush = [&](const float (&A)[8], const float X, const u32x4 s0, const u32x4 s1) {
+                // attention output merged from the split-KV partials {max, sum, o[hd]} per (head, split); the arithmetic of the
+                // 16-bit kernel's merge producer: pairwise-tree sum of the rescaled denominators, fmaf chain over the splits
+                const int hd = a.att_hd, hs = hd + 2;
+                auto merge = [&](auto ns_tag) {
+                    constexpr int NS = decltype(ns_tag)::value;
+                    float2 st[R][NS];
+                    float ov[R][NS];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const uint32_t pr = k < 4 ? s0[k] : s1[k - 4];  // bf16 pair: scale (low half), zero (high half)
-            const float sc = __uint_as_float(pr << 16), zr = __uint_as_float(pr & 0xFFFF0000u);
-            float t;
-            if constexpr (BF16) t = A[k] - 136.0f * X;                         // (128 + q) - 136
-            else if (k & 1) t = fmaf(A[k], 0.0625f, -72.0f * X);               // ((1024 + 16 q) - 1024) / 16 - 8
-            else t = A[k] - 1032.0f * X;                                       // (1024 + q) - 1032
-            total[k] += fmaf(sc, t, zr * X);
-        }
-    };
-    // unit u belongs to slice u % split, and inside the slice to wave (u / split) % 16
-    const int ustride = split * WAVES;
-    // phases 1 and 2 of a pass whose first unit is u0: activations, ballots, the wave's lists (li, lx); cnt[i] = kept pairs
-    auto front = [&](const int u0, uint8_t* li, uint32_t* lx, int (&cnt)[UP], bool (&live)[UP]) {
-        // ---- 1. activations of the pass ----------------------------------------------------------------------------------------
-        // The element-wise producers (MODE 2, MODE 4) run HERE, per unit, in the registers of the wave that owns the unit:
-        // a workgroup touches only its own slice of gate | up (of the attention partials), not the whole vector.
-        uint32_t xb[UP];
-        uint32_t m_el[UP];  // the lane's element of unit i (lanes 32..63 mirror 0..31)
+                    for (int j = 0; j < R; ++j) {
+                        const int m = (int)m_el[j];
+                        const int h = m / hd, d = m - h * hd;
+                        const float* b = a.att + (size_t)h * NS * hs;
 #pragma unroll
-        for (int i = 0; i < UP; ++i) {
-            const int u = u0 + i * ustride;
-            live[i] = u < nunits;  // wave-uniform
-            const int uu = live[i] ? u : u0;
-            m_el[i] = (uint32_t)(uu << 5) + (lane & 31);
-        }
-        if constexpr (MODE == 0) {
-#pragma unroll
-            for (int i = 0; i < UP; ++i) xb[i] = a.x[m_el[i]];
-        } else if constexpr (MODE == 1) {
-#pragma unroll
-            for (int i = 0; i < UP; ++i) xb[i] = xs[m_el[i]];
-        } else if constexpr (MODE == 2) {
-            // x = round(round(silu(gate)) * up)                                      gpt-fast/model.py:258-259
-            uint32_t gb[UP], ub[UP];
-#pragma unroll
-            for (int i = 0; i < UP; ++i) {  // all gate / up loads of the pass first
-                gb[i] = a.x[m_el[i]];
-                ub[i] = a.x[(uint32_t)Z + m_el[i]];
-            }
-#pragma unroll
-            for (int i = 0; i < UP; ++i) {
-                const float gt = bits_to_float(gb[i], BF16);
-                const float sl = bits_to_float(float_to_bits<BF16>(gt / (1.0f + expf(-gt))), BF16);
-                xb[i] = float_to_bits<BF16>(sl * bits_to_float(ub[i], BF16));
-            }
-        } else {
-            // attention output merged from the split-KV partials {max, sum, o[hd]} per (head, split); the arithmetic of the
-            // 16-bit kernel's merge producer: pairwise-tree sum of the rescaled denominators, fmaf chain over the splits
-            const int hd = a.att_hd, hs = hd + 2;
-            auto merge = [&](auto ns_tag, auto i0_tag, auto n_tag) {
-                constexpr int NS = decltype(ns_tag)::value, I0 = decltype(i0_tag)::value, NU = decltype(n_tag)::value;
-                float2 st[NU][NS];
-                float ov[NU][NS];
-#pragma unroll
-                for (int j = 0; j < NU; ++j) {
-                    const int m = (int)m_el[I0 + j];
-                    const int h = m / hd, d = m - h * hd;
-                    const float* b = a.att + (size_t)h * NS * hs;
-#pragma unroll
-                    for (int q = 0; q < NS; ++q) {
-                        st[j][q] = *reinterpret_cast<const float2*>(b + q * hs);
-                        ov[j][q] = b[q * hs + 2 + d];
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < NU; ++j) {
-                    float M = st[j][0].x;
-#pragma unroll
-                    for (int q = 1; q < NS; ++q) M = fmaxf(M, st[j][q].x);
-                    float f[NS], t[NS];
-#pragma unroll
-                    for (int q = 0; q < NS; ++q) {
-                        f[q] = st[j][q].y > 0.0f ? expf(st[j][q].x - M) : 0.0f;
-                        t[q] = st[j][q].y * f[q];
-                    }
-                    float Ls = (t[0] + t[1]) + (t[2] + t[3]);
-                    if constexpr (NS == 8) Ls = Ls + ((t[7] + t[6]) + (t[5] + t[4]));
-                    float Os = 0.0f;
-#pragma unroll
-                    for (int q = 0; q < NS; ++q) Os = fmaf(ov[j][q], f[q] / Ls, Os);
-                    xb[I0 + j] = float_to_bits<BF16>(Os);
-                }
-            };
-            using I = std::integral_constant<int, 0>;
-            if (a.att_ns == 8) {  // 24 registers of partials per unit: two units at a time
-                merge(std::integral_constant<int, 8>{}, I{}, std::integral_constant<int, 2>{});
-                if constexpr (UP == 4) merge(std::integral_constant<int, 8>{}, std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
-            } else {
-                merge(std::integral_constant<int, 4>{}, I{}, std::integral_constant<int, UP>{});
-            }
-        }
-        stamp(3);
-        // ---- 2. ballots -> kept row pairs of every unit in the wave's lists (16 slots per unit, ascending) -----------------
-#pragma unroll
-        for (int i = 0; i < UP; ++i) {
-            const float v = bits_to_float(xb[i], BF16);
-            const bool keep = keep_rule(v, tau) || (v != v);
-            const uint32_t mask = live[i] ? (uint32_t)__ballot(keep) : 0u;  // lanes 32..63 mirror 0..31
-            const uint32_t pm = (mask | (mask >> 1)) & 0x55555555u;          // bit 2p: pair p has a kept row
-            const uint32_t xm = keep ? xb[i] : 0u;
-            const uint32_t xn = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)xm, 0xB1, 0xf, 0xf, false);  // lane ^ 1
-            if (lane < 32 && ((pm >> lane) & 1u)) {  // even lanes of kept pairs
-                const uint32_t rank = __builtin_amdgcn_mbcnt_lo(pm, 0u);
-                const uint32_t slot = (uint32_t)i * 16u + (SHARE ? (rank & 3u) * 4u + (rank >> 2) : rank);
-                li[slot] = (uint8_t)(lane >> 1);
-                lx[slot] = xm | (xn << 16);
-            }
-            cnt[i] = __popc(pm);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-    for (int u0 = slice + split * wave; u0 < nunits; u0 += ustride * UP) {
-        int cnt[UP];  // kept pairs of unit i (wave-uniform)
-        bool live[UP];
-        front(u0, li, lx, cnt, live);
-        stamp(4);
-        if constexpr (SHARE) {
-            // ---- 3s. the four lane groups share each unit: group rs takes the pairs of rank rs, rs + 4, ... (<= 4 steps per unit)
-            u32x4 sz0[UP], sz1[UP];
-#pragma unroll
-            for (int i = 0; i < UP; ++i) {
-                const int uu = live[i] ? u0 + i * ustride : u0;  // wave-uniform
-                const u32x4* szp = reinterpret_cast<const u32x4*>(szb + (size_t)((uu << 5) >> a.gshift) * szld * 2);
-                sz0[i] = szp[0];
-                sz1[i] = szp[1];
-            }
-            u32x2 d[UP][4];
-#pragma unroll
-            for (int i = 0; i < UP; ++i) {
-                const uint32_t pidx = *reinterpret_cast<const uint32_t*>(li + i * 16 + rs * 4);  // the group's four pair indices
-                const uint32_t row_off = (uint32_t)((live[i] ? u0 + i * ustride : u0) << 4) * uldb + lane_off;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    d[i][r] = u32x2{0u, 0u};
-                    if (4 * r < cnt[i]) {          // wave-uniform: this step has pairs
-                        if (4 * r + rs < cnt[i])   // (a slot past the count holds a stale index: never dereferenced)
-                            d[i][r] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(wtile + (row_off + ((pidx >> (8 * r)) & 0xFFu) * uldb)));
-                    }
-                }
-            }
-            stamp(5);
-            // ---- 4s. arithmetic, unit by unit; scale / zero once per (unit, column) — linear, so every group applies them to
-            //          its own share and the shares meet in the reduce at the end of the kernel
-#pragma unroll
-            for (int i = 0; i < UP; ++i) {
-                if (i == 1) stamp(6);
-                float A[8], X = 0.0f;
-#pragma unroll
-                for (int k = 0; k < 8; ++k) A[k] = 0.0f;
-                const u32x4 xx4 = *reinterpret_cast<const u32x4*>(lx + i * 16 + rs * 4);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (4 * r < cnt[i]) {
-                        const uint32_t x2 = (4 * r + rs < cnt[i]) ? xx4[r] : 0u;  // a group without a pair adds 0
-                        mac16(d[i][r], x2, A, X);
-                    }
-                }
-                flush(A, X, sz0[i], sz1[i]);
-            }
-        } else {
-            // ---- 3. 16-lane group rs takes unit rs of the pass: its group parameters (32 bytes per lane, once) and every
-            //         pair-row load of its unit, one pair per step, all issued before the first is consumed ----------------------
-            const int cntv = rs == 0 ? cnt[0] : (rs == 1 ? cnt[1] : (rs == 2 ? cnt[2] : cnt[3]));
-            const int maxcnt = max(max(cnt[0], cnt[1]), max(cnt[2], cnt[3]));  // wave-uniform step count
-            const int uv = min(u0 + rs * ustride, nunits - 1);                 // (a dead unit has no pairs: any valid address)
-            const u32x4* szp = reinterpret_cast<const u32x4*>(szb + (size_t)((uv << 5) >> a.gshift) * szld * 2);
-            const u32x4 sz0 = szp[0], sz1 = szp[1];
-            const uint32_t row_off = (uint32_t)(uv << 4) * uldb + lane_off;  // first pair-row of the group's unit
-            u32x2 d[16];
-            {
-                const u32x4 pidx = *reinterpret_cast<const u32x4*>(li + rs * 16);  // the group's 16 pair indices
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    d[r] = u32x2{0u, 0u};
-                    if (r < maxcnt) {     // wave-uniform
-                        if (r < cntv)     // (a slot past the count holds a stale index: never dereferenced)
-                            d[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(wtile + (row_off + ((pidx[r >> 2] >> (8 * (r & 3))) & 0xFFu) * uldb)));
-                    }
-                }
-            }
-            stamp(5);
-            // ---- 4. arithmetic; scale / zero once per (unit, column) ---------------------------------------------------------------
-            {
-                float A[8], X = 0.0f;
-#pragma unroll
-                for (int k = 0; k < 8; ++k) A[k] = 0.0f;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if (q == 1) stamp(6);
-                    if (q * 4 < maxcnt) {
-                        const u32x4 xx4 = *reinterpret_cast<const u32x4*>(lx + rs * 16 + q * 4);
-#pragma unroll
-                        for (int rr = 0; rr < 4; ++rr) {
-                            const int r = q * 4 + rr;
-                            if (r < maxcnt) {
-                                const uint32_t x2 = (r < cntv) ? xx4[rr] : 0u;  // a group past its count adds 0
-                                    mac16(d[r], x2, A, X);
-                            }
+                        for (int q = 0; q < NS; ++q) {
+                            st[j][q] = *reinterpret_cast<const float2*>(b + q * hs);
+                            ov[j][q] = b[q * hs + 2 + d];
                         }
                     }
-                }
-                    flush(A, X, sz0, sz1);
+#pragma unroll
+                    for (int j = 0; j < R; ++j) {
+                        float M = st[j][0].x;
+#pragma unroll
+                        for (int q = 1; q < NS; ++q) M = fmaxf(M, st[j][q].x);
+                        float f[NS], t[NS];
+#pragma unroll
+                        for (int q = 0; q < NS; ++q) {
+                            f[q] = st[j][q].y > 0.0f ? expf(st[j][q].x - M) : 0.0f;
+                            t[q] = st[j][q].y * f[q];
+                        }
+                        float Ls = (t[0] + t[1]) + (t[2] + t[3]);
+                        if constexpr (NS == 8) Ls = Ls + ((t[7] + t[6]) + (t[5] + t[4]));
+                        float Os = 0.0f;
+#pragma unroll
+                        for (int q = 0; q < NS; ++q) Os = fmaf(ov[j][q], f[q] / Ls, Os);
+                        xb[j] = float_to_bits<BF16>(Os);
+                    }
+                };
+                if (a.att_ns == 8) merge(std::integral_constant<int, 8>{});
+                else merge(std::integral_constant<int, 4>{});
             }
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+                if (e0 + 1024 * i < total) xs[e0 + 1024 * i] = masked(xb[i]);
         }
-        stamp(7);
-        first_pass = false;
-        __builtin_amdgcn_wave_barrier();  // the lists are rewritten by the next pass
+        if (tid < 32) xs[total + tid] = 0;
+        __syncthreads();
     }
-    first_pass = true;
+    stamp(3);
+    // ---- the stream ----------------------------------------------------------------------------------------------------------
+    const uint32_t uldb = (uint32_t)ldb, col = (uint32_t)(tile - seg_tile0) * BN;
+    const RowsBuf wbuf = rows_buffer(reinterpret_cast<const uint16_t*>(seg_wq + col), (size_t)(Z / 2 - 1) * ldb + BN);
+    const RowsBuf pbuf = rows_buffer(seg_sz + 2 * (size_t)col, (size_t)((Z >> a.gshift) - 1) * szld * 4 + BN * 4);
+    constexpr uint32_t kBias = BF16 ? 0x43004300u : 0x64006400u;  // (128, 128) bf16 / (1024, 1024) fp16
+    constexpr uint32_t kOnes = BF16 ? 0x3F803F80u : 0x3C003C00u;  // (1, 1)
+    struct Unit {
+        u32x4 x;     // the lane's eight masked activations (rows 8 g ..)
+        u32x2 w[4];  // its four pairs
+        u32x2 p;     // (scale, zero) of columns 8 cl + 2 g and the next
+    } st[DEPTH];
+    // (units past the last read the zeros behind the activations, so nothing is requested for them; no branch: the loads in flight are counted)
+    const int xpast = MODE == 1 ? Z : nk * 32;
+    auto read_x = [&](const int k) {
+        const int at = MODE == 1 ? (slice + split * k) << 5 : k << 5;
+        return *reinterpret_cast<const u32x4*>(xs + (k < nk ? at : xpast) + 8 * g);
+    };
+    uint32_t loff[4];  // the lane's pair i inside a unit
+#pragma unroll
+    for (int i = 0; i < 4; ++i) loff[i] = (uint32_t)(4 * g + i) * uldb + 8u * (uint32_t)cl;
+    const uint32_t poff = 32u * (uint32_t)cl + 8u * (uint32_t)g;
+    auto request = [&](Unit& t, const int k) {
+        const int u = slice + split * min(k, nk - 1);
+        t.x = read_x(k);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) t.w[i] = __builtin_amdgcn_raw_buffer_load_b64(wbuf, (int)(t.x[i] ? loff[i] : kRowsNowhere), (int)((uint32_t)u * 16u * uldb), 2);
+        t.p = __builtin_amdgcn_raw_buffer_load_b64(pbuf, (int)poff, (int)(((uint32_t)(u << 5) >> a.gshift) * (uint32_t)szld * 4u), 0);
+    };
+    u32x4 ones = {kOnes, kOnes, kOnes, kOnes};
+    uint32_t bias = kBias;
+    asm volatile("" : "+v"(ones), "+v"(bias));  // (kept in registers: with a literal the mask-and-or would be two instructions)
+    // Lane group g finishes columns 2 g, 2 g + 1 of the lane's eight, so the product of column j is wanted in the rows 4 (j / 2) .. of the
+    // result only: the first operand is x in the lanes of those rows and zeros in the others — read from the zeros behind the
+    // activations —, and the even and the odd columns each add up in one accumulator, no selection afterwards
+    const int bank = cl >> 2;
+    float total0 = 0.0f, total1 = 0.0f;
+    auto consume = [&](const Unit& t, const int k) {
+        const int at = MODE == 1 ? (slice + split * k) << 5 : k << 5;
+        f32x4 even = {0.f, 0.f, 0.f, 0.f}, odd = even;
+        u32x4 xb[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) xb[q] = *reinterpret_cast<const u32x4*>(xs + (bank == q ? at : xpast) + 8 * g);
+        const float X = mfma16<BF16>(t.x, ones, even)[0];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int h = q >> 1;
+            u32x4 be, bo;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t w = t.w[i][h];
+                if constexpr (BF16) {
+                    be[i] = ((q & 1 ? w >> 8 : w) & 0x000F000Fu) | bias;
+                    bo[i] = ((q & 1 ? w >> 12 : w >> 4) & 0x000F000Fu) | bias;
+                } else {
+                    const uint32_t v = q & 1 ? w >> 8 : w;
+                    be[i] = (v & 0x000F000Fu) | bias;
+                    bo[i] = (v & 0x00F000F0u) | bias;  // 1024 + 16 q
+                }
+            }
+            even = mfma16<BF16>(xb[q], be, even);
+            odd = mfma16<BF16>(xb[q], bo, odd);
+        }
+        const float s0 = __uint_as_float(t.p[0] << 16), z0 = __uint_as_float(t.p[0] & 0xFFFF0000u), s1 = __uint_as_float(t.p[1] << 16), z1 = __uint_as_float(t.p[1] & 0xFFFF0000u);
+        // sum x (q - 8) from the biased sums
+        const float t0 = fmaf(BF16 ? -136.0f : -1032.0f, X, even[0]), t1 = BF16 ? fmaf(-136.0f, X, odd[0]) : fmaf(odd[0], 0.0625f, -72.0f * X);
+        total0 += fmaf(s0, t0, z0 * X);
+        total1 += fmaf(s1, t1, z1 * X);
+    };
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) request(st[i], wave + WAVES * i);
+    stamp(5);
+    int k = wave;
+    for (; k + WAVES * (DEPTH - 1) < nk; k += WAVES * DEPTH) {
+#pragma unroll
+        for (int i = 0; i < DEPTH; ++i) {
+            consume(st[i], k + WAVES * i);
+            __builtin_amdgcn_sched_barrier(0);
+            request(st[i], k + WAVES * (DEPTH + i));
+        }
+        if (k == wave) stamp(6);
+    }
+#pragma unroll
+    for (int i = 0; i < DEPTH - 1; ++i)
+        if (k + WAVES * i < nk) consume(st[i], k + WAVES * i);
     stamp(8);
-    // ---- reduce: the four row groups of the wave, then the waves in fixed order -------------------------------------------
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        total[k] = xor_add<16>(total[k]);
-        total[k] = xor_add<32>(total[k]);
-    }
-    if (lane < 16) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) red[wave * BN + lane * 8 + k] = total[k];
-    }
+    // ---- reduce: the waves in fixed order ------------------------------------------------------------------------------------
+    *reinterpret_cast<float2*>(red + wave * BN + 8 * cl + 2 * g) = make_float2(total0, total1);
     __syncthreads();
     stamp(9);
     const uint32_t c = (uint32_t)tile * BN + tid;  // column in the concatenation of the segments (slab / partial index)
@@ -520,16 +404,26 @@ __global__ __launch_bounds__(1024) void sparse_gemv_int4_kernel(const I4Args a) 
     }
 }
 
-template <bool BF16, int KIND, bool PHASE>
+template <bool BF16, bool PHASE>
 static hipError_t launch_i4(const I4Args& a, int mode, dim3 grid, size_t lds, hipStream_t st) {
     const dim3 block(1024);
     switch (mode) {
-        case TEAL_IN_PLAIN: hipLaunchKernelGGL((sparse_gemv_int4_kernel<BF16, 0, KIND, PHASE>), grid, block, 0, st, a); break;
-        case TEAL_IN_RESID_NORM: hipLaunchKernelGGL((sparse_gemv_int4_kernel<BF16, 1, KIND, PHASE>), grid, block, lds, st, a); break;
-        case TEAL_IN_SILU_MUL: hipLaunchKernelGGL((sparse_gemv_int4_kernel<BF16, 2, KIND, PHASE>), grid, block, 0, st, a); break;
-        default: hipLaunchKernelGGL((sparse_gemv_int4_kernel<BF16, 4, KIND, PHASE>), grid, block, 0, st, a); break;
+        case TEAL_IN_PLAIN: hipLaunchKernelGGL((sparse_gemv_int4_kernel<BF16, 0, PHASE>), grid, block, lds, st, a); break;
+        case TEAL_IN_RESID_NORM: hipLaunchKernelGGL((sparse_gemv_int4_kernel<BF16, 1, PHASE>), grid, block, lds, st, a); break;
+        case TEAL_IN_SILU_MUL: hipLaunchKernelGGL((sparse_gemv_int4_kernel<BF16, 2, PHASE>), grid, block, lds, st, a); break;
+        default: hipLaunchKernelGGL((sparse_gemv_int4_kernel<BF16, 4, PHASE>), grid, block, lds, st, a); break;
     }
     return hipGetLastError();
+}
+
+// vectors beyond 28672 rows a slice need more LDS than a kernel gets unasked (first use of a device, device_ctx())
+bool int4_device_init() {
+    bool ok = true;
+#define TEAL_OPT(BF, M) ok = ok && hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse_gemv_int4_kernel<BF, M>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kI4MaxLds) == hipSuccess
+    TEAL_OPT(false, 0); TEAL_OPT(false, 1); TEAL_OPT(false, 2); TEAL_OPT(false, 4); TEAL_OPT(true, 0); TEAL_OPT(true, 1); TEAL_OPT(true, 2); TEAL_OPT(true, 4);
+#undef TEAL_OPT
+    if (!ok) (void)hipGetLastError();
+    return ok;
 }
 
 // One launch over int4 weights: [producer] -> mask + compaction -> gathered GEMV over every segment (teal_fused_gemv with
@@ -593,7 +487,7 @@ int fused_gemv_i4(const teal_gemv_in_t* in, const teal_gemv_out_t* out, int Z, i
             a.norm_w = reinterpret_cast<const uint16_t*>(in->norm_weight);
             a.eps = in->eps;
             a.resid_out = reinterpret_cast<uint16_t*>(in->resid_out);
-            lds = (size_t)Z * 2;
+            lds = (size_t)Z * 2 + 64;
             break;
         default: return TEAL_ERR_ARG;  // TEAL_IN_MASKED: no int4 form
     }
@@ -618,29 +512,25 @@ int fused_gemv_i4(const teal_gemv_in_t* in, const teal_gemv_out_t* out, int Z, i
         }
     }
     const dim3 grid(ntiles, split);
-    // a wave's units: up to two -> its lane groups share each unit; more -> passes of four, a unit per lane group
-    const int upw = (nunits + split * 16 - 1) / (split * 16);
-    const int kind = upw <= 2 ? kI4Share : kI4Group;
+    if (in->mode != TEAL_IN_RESID_NORM) lds = (size_t)((nunits + split - 1) / split) * 64 + 64;
+    if (lds > 56 * 1024 && !dc->int4_lds_ok) return TEAL_ERR_LAUNCH;
     hipError_t e;
-#define TEAL_I4_LAUNCH(BF, PH) \
-    (kind == kI4Share ? launch_i4<BF, kI4Share, PH>(a, in->mode, grid, lds, st) : launch_i4<BF, kI4Group, PH>(a, in->mode, grid, lds, st))
 #ifdef TEAL_DIAGNOSTICS
     if (g_phase && dtype == TEAL_F16) {  // measurement: the stamping instantiation (fp16 only; libteal_hip_diag.so)
         a.phase = phase_next_region();
-        e = TEAL_I4_LAUNCH(false, true);
+        e = launch_i4<false, true>(a, in->mode, grid, lds, st);
     } else
 #endif
     if (dtype == TEAL_BF16) {
-        e = TEAL_I4_LAUNCH(true, false);
+        e = launch_i4<true, false>(a, in->mode, grid, lds, st);
     } else {
-        e = TEAL_I4_LAUNCH(false, false);
+        e = launch_i4<false, false>(a, in->mode, grid, lds, st);
     }
-#undef TEAL_I4_LAUNCH
     if (e != hipSuccess) return TEAL_ERR_LAUNCH;
     if (out->desc || kDiagnostics) {
         char d[160];
-        snprintf(d, sizeof d, "sparse_gemv_int4_kernel<%s,%d,%d,false> grid (%d,%d) x 1024", dtype == TEAL_BF16 ? "true" : "false",
-                 in->mode, kind, ntiles, split);
+        snprintf(d, sizeof d, "sparse_gemv_int4_kernel<%s,%d,false> grid (%d,%d) x 1024", dtype == TEAL_BF16 ? "true" : "false",
+                 in->mode, ntiles, split);
         publish_desc(d, out->desc, out->desc_bytes);
     }
     if (nslabs_out) *nslabs_out = split;

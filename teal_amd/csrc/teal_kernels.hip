@@ -155,6 +155,7 @@ DeviceCtx* device_ctx() {
     }
     c->gqa_lds_ok = attention_device_init();
     c->prefill_lds_ok = prefill_device_init();
+    c->int4_lds_ok = int4_device_init();
     c->rows_lds_ok = rows_device_init();
     c->num_cu = cu;
     return c;
