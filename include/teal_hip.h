@@ -443,6 +443,14 @@ typedef struct teal_rows_gemm {
 int teal_rows_split(int M, int K, int N, int paired);
 int teal_rows_gemm(const teal_rows_gemm_t* args, int dtype, void* stream);
 
+/* ---- matrix products over a prompt's rows, teal_amd/csrc/teal_tile.hip -------------------------------------------------
+ * The same product for any number of rows: x [M][ldx] times one W^T image [K][ld], or two of one shape (gate and up); K % 64 == 0, N % 16 == 0.
+ * Results 16-bit y0 / y1 [M][ldy] (ldy % 8 == 0), or (slabs given, one image) the fp32 partial sums [teal_tile_split()][M][N]. */
+/* slices of K such a launch takes (1 without slabs); 0: not a case for it (the shape, or a vendor library is faster) */
+int teal_tile_split(int M, int K, int N, int images, int slabs);
+int teal_tile_gemm(const void* x, int ldx, const void* w0, const void* w1, int ld, void* y0, void* y1, int ldy, float* slabs, int M, int K, int N, int dtype,
+                   void* stream);
+
 /* ---- layered decoder designs: row kernels around their matrix products, teal_amd/csrc/teal_layered.hip ----------------
  * dtype 0 / 1 / 2 (fp16, bf16, fp32) = activations and weights; the residual stream is always fp32. */
 

@@ -21,7 +21,7 @@ CSRC = os.path.join(_PKG, "csrc")
 # (weight width, activation dtype) so that they compile in parallel
 SOURCES = ("teal_kernels.hip", "teal_attention.hip", "teal_gemv_w16_f16.hip", "teal_gemv_w16_bf16.hip",
            "teal_gemv_w8_f16.hip", "teal_gemv_w8_bf16.hip", "teal_gemv_fast_f16.hip", "teal_gemv_fast_bf16.hip", "teal_gemv_int4.hip",
-           "teal_gemv_fast_w8_f16.hip", "teal_gemv_fast_w8_bf16.hip", "teal_comparators.hip", "teal_prefill.hip", "teal_rows.hip", "teal_prompt.hip", "teal_layered.hip", "teal_latent.hip",
+           "teal_gemv_fast_w8_f16.hip", "teal_gemv_fast_w8_bf16.hip", "teal_comparators.hip", "teal_prefill.hip", "teal_rows.hip", "teal_tile.hip", "teal_prompt.hip", "teal_layered.hip", "teal_latent.hip",
            "teal_prompt_attention_capped.hip", "teal_grouped.hip", "teal_wkv.hip")
 # translation units whose kernels take their hot arguments as scalar parameters: the command processor preloads the
 # first 11 dwords into SGPRs at wave launch (no scalar-cache miss before the first activation load)
@@ -57,7 +57,7 @@ DIAG_LIB_PATH = os.path.join(_PKG, "libteal_hip_diag.so")
 # lacks are tolerated (OPTIONAL_WITH_OVERRIDE).
 LIB_OVERRIDE = os.environ.get("TEAL_LIB_PATH") or None
 OPTIONAL_WITH_OVERRIDE = ("teal_decode_attention_split_roped", "teal_prefill_gemm", "teal_prefill_resid_norm", "teal_prefill_attention",
-                          "teal_rows_split", "teal_rows_gemm", "teal_layer_resid_norm_slabs", "teal_prompt_norm", "teal_prompt_rope", "teal_prompt_attention", "teal_silu_mul",
+                          "teal_rows_split", "teal_rows_gemm", "teal_tile_split", "teal_tile_gemm", "teal_layer_resid_norm_slabs", "teal_prompt_norm", "teal_prompt_rope", "teal_prompt_attention", "teal_silu_mul",
                           "teal_layer_resid_norm", "teal_gated_act", "teal_logit_softcap", "teal_sample_rows", "teal_latent_prompt_rows", "teal_latent_gather",
                           "teal_layer_prompt_tile", "teal_layer_prompt_attention", "teal_latent_step_query", "teal_layer_step_attention",
                           "teal_latent_step_merge", "teal_grouped_prompt_rows", "teal_grouped_gather", "teal_grouped_step_attention", "teal_grouped_step_query", "teal_grouped_step_merge",
@@ -71,7 +71,7 @@ EXPORTS = (
     "teal_workspace_init", "teal_workspace_release", "teal_sample_topk_ws", "teal_decode_attention_split_ws", "teal_cmp_flag_gemv",
     "teal_decode_attention_split_roped",
     "teal_prefill_gemm", "teal_prefill_resid_norm", "teal_prefill_attention",
-    "teal_rows_split", "teal_rows_gemm", "teal_layer_resid_norm_slabs", "teal_prompt_norm", "teal_prompt_rope", "teal_prompt_attention", "teal_silu_mul",
+    "teal_rows_split", "teal_rows_gemm", "teal_tile_split", "teal_tile_gemm", "teal_layer_resid_norm_slabs", "teal_prompt_norm", "teal_prompt_rope", "teal_prompt_attention", "teal_silu_mul",
     "teal_layer_resid_norm", "teal_gated_act", "teal_logit_softcap", "teal_sample_rows",
     "teal_latent_prompt_rows", "teal_latent_gather", "teal_layer_prompt_tile", "teal_layer_prompt_attention",
     "teal_latent_step_query", "teal_layer_step_attention", "teal_latent_step_merge",
@@ -206,6 +206,8 @@ def _open(path: str, diag: bool) -> ctypes.CDLL:
     if hasattr(L, "teal_rows_gemm"):
         L.teal_rows_split.argtypes = [ci, ci, ci, ci]
         L.teal_rows_gemm.argtypes = [vp, ci, vp]
+        L.teal_tile_split.argtypes = [ci, ci, ci, ci, ci]
+        L.teal_tile_gemm.argtypes = [vp, ci, vp, vp, ci, vp, vp, ci, vp, ci, ci, ci, ci, vp]
         L.teal_layer_resid_norm_slabs.argtypes = [vp, ci, ci, vp, vp, ci, vp, ci, ci, ci, vp, vp, vp, cf, cf, vp, vp, vp, ci, ci, vp]
     if hasattr(L, "teal_prompt_norm"):
         L.teal_prompt_norm.argtypes = [vp, ci, vp, ci, vp, vp, vp, ci, vp, vp, ci, ci, cf, vp, ci, ci, vp]

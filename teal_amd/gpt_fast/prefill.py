@@ -173,8 +173,8 @@ class PrefillEngine:
 class PromptPass:
     """The prompt pass of any length for a patched 16-bit model: what Transformer.forward runs for more than one token (model.fused_decode), in
     place of some thirty launches per layer of the op-by-op modules.  Per layer: norm -> wqkv -> rotation and cache rows -> attention over the cache ->
-    wo -> norm -> gate | up, silu * up -> down (csrc/teal_prompt.hip; products over up to 64 rows by csrc/teal_rows.hip, larger ones by the vendor
-    library).  Dense, same rounding points, same results: logits [1, T, vocab] of every token.  Holds no state of its own."""
+    wo -> norm -> gate | up, silu * up -> down (csrc/teal_prompt.hip; products over up to 64 rows by csrc/teal_rows.hip, over some hundred by
+    csrc/teal_tile.hip where that is faster, others by the vendor library).  Dense, same rounding points, same results: logits [1, T, vocab] of every token.  Holds no state of its own."""
 
     @staticmethod
     def supports(model: Transformer) -> Optional[str]:
@@ -246,7 +246,7 @@ class PromptPass:
             norm(layer.ffn_norm.weight, K.linear(at.wo, y, tickets, slabs=True))
             mid = K.gated_pair(ff.w1, ff.w3, x, "silu_rounded", tickets)
             if mid is None:
-                gate, up = K.linear(ff.w1, x, tickets), K.linear(ff.w3, x, tickets)
+                gate, up = K.both(ff.w1, ff.w3, x)
                 mid = gate  # (in place)
                 _lib.check(L.teal_silu_mul(gate.data_ptr(), up.data_ptr(), mid.data_ptr(), mid.numel(), code, st), "teal_silu_mul")
             norm(layers[i + 1].attention_norm.weight if i + 1 < len(layers) else m.norm.weight, K.linear(ff.w2, mid, tickets, slabs=True))

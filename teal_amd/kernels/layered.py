@@ -55,17 +55,34 @@ def rows_weight(lin) -> Optional[torch.Tensor]:
     return lin.weight
 
 
+def _image(x, w) -> bool:
+    """x [M, K] and the column-major w [N, K] as the products' kernels take them: one 16-bit type, aligned, in reach of a 32-bit offset"""
+    return (w.dtype in (torch.float16, torch.bfloat16) and x.dtype == w.dtype and w.is_cuda and w.stride(0) == 1 and w.stride(1) >= w.shape[0] and not w.stride(1) & 7
+            and x.stride(1) == 1 and not x.stride(0) & 7 and not (w.data_ptr() | x.data_ptr()) & 15 and w.shape[1] * w.stride(1) * 2 <= 0xFFF00000)
+
+
 def rows_split(x, w, paired: bool = False) -> int:
     """slices teal_rows_gemm takes for x [M, K] and the column-major w [N, K]; 0: not a case for it"""
     M, (N, Kd) = x.shape[0], w.shape
     if paired:
         N //= 2
-    if (M > (ROWS_PAIR_MAX if paired else ROWS_MAX) or w.dtype not in (torch.float16, torch.bfloat16) or x.dtype != w.dtype or not w.is_cuda or w.stride(0) != 1
-            or w.stride(1) < w.shape[0] or w.stride(1) & 7 or x.stride(1) != 1 or x.stride(0) & 7 or (w.data_ptr() | x.data_ptr()) & 15):
-        return 0
-    if (N & 7) or Kd * w.stride(1) * 2 > 0xFFF00000:
+    if M > (ROWS_PAIR_MAX if paired else ROWS_MAX) or (N & 7) or not _image(x, w):
         return 0
     return int(_lib.load().teal_rows_split(M, Kd, N, int(paired)))
+
+
+def tile_split(x, w, images: int = 1, slabs: bool = False) -> int:
+    """slices teal_tile_gemm takes for more rows than teal_rows_gemm does (w: one of `images` of its shape); 0: not a case for it"""
+    M, (N, Kd) = x.shape[0], w.shape
+    if M <= ROWS_MAX or not _image(x, w) or x.stride(0) < Kd or M * x.stride(0) * 2 > 0xFFF00000:
+        return 0
+    return int(_lib.load().teal_tile_split(M, Kd, N, images, int(slabs)))
+
+
+def _tile_gemm(x, w, N, y, y_up=None, w_up=None, slabs=False):
+    _run("teal_tile_gemm", x.data_ptr(), x.stride(0), w.data_ptr(), w_up, w.stride(1), None if slabs else y.data_ptr(), _p(y_up), y.stride(-2), y.data_ptr() if slabs else None,
+         x.shape[0], w.shape[1], N, runtime.dtype_code(x.dtype))
+    return y
 
 
 def _rows_gemm(x, w, N, split, mode, tickets, y, w_up=None, bias=None, bias_up=None, act=-1, n_valid=0, softcap=0.0):
@@ -81,7 +98,10 @@ def _rows_gemm(x, w, N, split, mode, tickets, y, w_up=None, bias=None, bias_up=N
 
 def linear(lin, x, tickets=None, slabs: bool = False, weight=None, act: Optional[str] = None, bias=None):
     """act(x W^T + bias) of a linear (or of rows of its weight).  With `tickets` (zero counters, left zero: one set per pass) a few rows go through
-    teal_rows_gemm; `slabs`: the result may then be the product's fp32 partial sums [slices, rows, columns] instead, for resid_norm to add"""
+    teal_rows_gemm; `slabs`: the result may be the product's fp32 partial sums [slices, rows, columns] instead (of a few rows, or teal_tile_gemm's of
+    more), for resid_norm to add"""
+    if slabs and act is None and weight is None and x.shape[0] > ROWS_MAX and (w := rows_weight(lin)) is not None and (split := tile_split(x, w, slabs=True)):
+        return _tile_gemm(x, w, w.shape[0], torch.empty(split, x.shape[0], w.shape[0], device=x.device, dtype=torch.float32), slabs=True)
     w = (rows_weight(lin) if tickets is not None else None) if weight is None else weight
     split = rows_split(x, w) if w is not None and tickets is not None else 0
     if split == 0:
@@ -99,6 +119,10 @@ def gated_linear(lin, x, act: str, bias=None, tickets=None):
     N = lin.out_features // 2
     split = rows_split(x, w, True) if w is not None and not N & 63 else 0
     if split == 0:
+        w = rows_weight(lin) if x.shape[0] > ROWS_MAX else None
+        if w is not None and not N & 7 and tile_split(x, w[:N], 2):
+            gu = torch.empty(x.shape[0], 2 * N, device=x.device, dtype=x.dtype)
+            return gated_act(_tile_gemm(x, w, N, gu, gu[:, N:], w.data_ptr() + 2 * N), N, N, act, bias)
         return gated_act(lin(x), N, N, act, bias)
     y = torch.empty(x.shape[0], N, device=x.device, dtype=x.dtype)
     return _rows_gemm(x, w, N, split, ROWS_ROUNDED, tickets, y, w_up=w.data_ptr() + 2 * N, bias=None if bias is None else bias[:N], bias_up=None if bias is None else bias[N:],
@@ -114,6 +138,16 @@ def gated_pair(gate, up, x, act: str, tickets=None):
         return None
     split = int(_lib.load().teal_rows_split(x.shape[0], w.shape[1], w.shape[0], 1))
     return _rows_gemm(x, w, w.shape[0], split, ROWS_ROUNDED, tickets, torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype), w_up=u.data_ptr(), act=ACTS[act])
+
+
+def both(gate, up, x):
+    """(gate(x), up(x)) of two linears"""
+    w, u = rows_weight(gate), rows_weight(up)
+    if w is None or u is None or w.shape != u.shape or w.stride() != u.stride() or u.dtype != w.dtype or u.data_ptr() & 15 or not tile_split(x, w, 2):
+        return gate(x), up(x)
+    y = torch.empty(2, x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
+    _tile_gemm(x, w, w.shape[0], y[0], y[1], u.data_ptr())
+    return y[0], y[1]
 
 
 def head(lin, h, vocab: int, cap: Optional[float], tickets=None):

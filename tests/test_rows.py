@@ -147,3 +147,69 @@ def test_resid_norm_adds_slabs(D):
     h = Kn.resid_norm(got, y=y, post_w=post, pre_w=pre, eps=1e-5, rows=rows, zero=zero)
     assert torch.allclose(got[rows.long()], want[rows.long()], atol=1e-5, rtol=1e-5) and torch.equal(got[0], x[0]) and not zero.any()
     assert torch.allclose(h.float(), (norm(want) * pre.float())[rows.long()], atol=1e-2, rtol=2 ** -7)
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("M,K,N", [(1, 64, 16), (47, 256, 272), (65, 320, 2064), (161, 4096, 496), (320, 11008, 256), (640, 2048, 1024)])
+def test_tile_gemm(M, K, N, dtype):
+    """every output of teal_tile_gemm: part tiles of rows and columns, one slice and several (unequal ones), one image and two, rows of x, of the
+    images and of y further apart than their columns; nothing outside the result is written"""
+    from teal_amd import _lib, runtime
+    L, dt = _lib.load(), DT[dtype]
+    runtime.init()
+    g = torch.Generator(device=DEV).manual_seed(K + M)
+    x = torch.full((M, K + 8), float("nan"), device=DEV, dtype=dt)
+    x[:, :K] = torch.randn(M, K, device=DEV, generator=g).to(dt)
+    img = _image(K, 2 * N, dtype, 3)
+    y = torch.full((M + 1, 2 * N + 8), 7.0, device=DEV, dtype=dt)
+
+    def run(images, slabs):
+        up = images == 2
+        rc = L.teal_tile_gemm(x.data_ptr(), K + 8, img.data_ptr(), img.data_ptr() + 2 * N if up else None, img.stride(0), None if slabs is not None else y.data_ptr(),
+                              y.data_ptr() + 2 * N if up else None, y.stride(0), None if slabs is None else slabs.data_ptr(), M, K, N, dtype, runtime.stream_ptr())
+        assert rc == 0
+
+    def rounded(cols):
+        want = (x[:, :K].double() @ img[:, :cols].double())
+        err, size = (y[:M, :cols].double() - want).abs(), x[:, :K].double().abs() @ img[:, :cols].double().abs()
+        assert bool((err <= 2.0 ** -18 * size + 2.0 ** (-11 if dtype == 0 else -8) * want.abs() + 2.0 ** -25).all())
+        assert bool((y[:M, cols:] == 7).all()) and bool((y[M] == 7).all())
+
+    run(1, None)
+    rounded(N)
+    run(2, None)
+    rounded(2 * N)
+    if (split := L.teal_tile_split(M, K, N, 1, 1)) > 0:
+        slabs = torch.full((split + 1, M, N), float("nan"), device=DEV)
+        run(1, slabs)
+        assert bool(slabs[split].isnan().all())
+        _close(slabs[:split].sum(0), x[:, :K].float(), img[:, :N].float(), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_tile_products_of_linears(dtype):
+    """the linears of a prompt by either route: partial sums, gate and up apart and as one matrix; others (a hook, a bias) keep the module's"""
+    from teal_amd import runtime
+    from teal_amd.kernels import layered as Kn
+    from teal_amd.monkeypatch import to_column_major
+    runtime.init()
+    torch.manual_seed(0)
+
+    def lin(n, k, w=None):
+        m = torch.nn.Linear(k, n, bias=False, device=DEV, dtype=dtype)
+        m.weight.data = (torch.randn(n, k, device=DEV) * k ** -0.5).to(dtype) if w is None else w
+        to_column_major(m)
+        return m
+
+    step = 2.0 ** (-10 if dtype is torch.float16 else -7)
+    x, down, gate, up = torch.randn(100, 1024, device=DEV).to(dtype), lin(512, 1024), lin(8192, 1024), lin(8192, 1024)
+    y = Kn.linear(down, x, slabs=True)
+    assert y.dim() == 3 and y.dtype == torch.float32
+    assert (y.sum(0) - x.float() @ down.weight.float().T).abs().max() < 1e-4  # (sums of 1024 products near 1)
+    wide = lin(16384, 1024, torch.cat([gate.weight, up.weight]))
+    got = Kn.gated_linear(wide, x, "silu")
+    for a, lin_ in zip(Kn.both(gate, up, x), (gate, up)):
+        assert (a.float() - x.float() @ lin_.weight.float().T).abs().max() < 4 * step
+    assert torch.equal(got, Kn.gated_act(torch.cat(Kn.both(gate, up, x), 1), 8192, 8192, "silu"))
+    down.register_forward_hook(lambda *a: None)
+    assert Kn.linear(down, x, slabs=True).dim() == 2
