@@ -205,6 +205,12 @@ __device__ __forceinline__ uint32_t order_key32(const float f) {
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
+// Bound by latency: five or so passes of one workgroup over its row.  PIECES > 0: the row is read once, 16 bytes at a time, and stays in registers
+// (1024 x 4 PIECES logits; with 16 pieces the compiler does not keep them there: 65536 logits 167 us, from memory 60); 0: any size, stride and
+// alignment, every pass reads memory.  32000 logits, top 200: 46 us from memory, 21 from registers; 8000: 19 and 12.
+__device__ __forceinline__ float from_order_key32(const uint32_t k) { return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k); }
+
+template <int PIECES>
 __global__ __launch_bounds__(1024) void sample_rows_kernel(const float* __restrict__ logits, const int ld, const int V, const int top_k, const float inv_temp,
                                                            unsigned long long* __restrict__ rng, int32_t* __restrict__ token_out, int32_t* __restrict__ pos_inout,
                                                            int32_t* __restrict__ history, const int history_len) {
@@ -213,10 +219,45 @@ __global__ __launch_bounds__(1024) void sample_rows_kernel(const float* __restri
     __shared__ int ired[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row = blockIdx.x;
     const float* x = logits + (size_t)row * ld;
+    u32x4 own[PIECES > 0 ? PIECES : 1];  // logits, then their distances d from the largest: one register each, whatever a pass wants of them
     float mx = -INFINITY;
-    for (int i = tid; i < V; i += 1024) mx = fmaxf(mx, x[i]);
+    if constexpr (PIECES > 0) {
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) own[p] = *reinterpret_cast<const u32x4*>(x + min(4 * (1024 * p + tid), V - 4));
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {  // (past the end: the last logits once more)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) mx = fmaxf(mx, __uint_as_float(own[p][j]));
+        }
+    } else {
+        for (int i = tid; i < V; i += 1024) mx = fmaxf(mx, x[i]);
+    }
     mx = block_max<1024>(mx, fred, tid);
     const uint32_t kmax = order_key32(mx);
+    if constexpr (PIECES > 0) {
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                own[p][j] = kmax - order_key32(__uint_as_float(own[p][j]));
+                asm volatile("" : "+v"(own[p][j]));  // (or both forms are kept)
+            }
+        }
+    }
+    auto each = [&](auto f) {  // f(index, d) for the thread's logits
+        if constexpr (PIECES > 0) {
+#pragma unroll
+            for (int p = 0; p < PIECES; ++p) {
+                const int i = 4 * (1024 * p + tid);
+                if (i < V) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) f(i + j, own[p][j]);
+                }
+            }
+        } else {
+            for (int i = tid; i < V; i += 1024) f(i, kmax - order_key32(x[i]));
+        }
+    };
     uint32_t limit = 0xFFFFFFFFu;  // keep keys with kmax - key <= limit
     if (top_k > 0 && top_k < V && inv_temp > 0.0f) {
         // histogram of (d - lo) >> sh for d in [lo, lo + (256 << sh)); leaves the bin of the need-th key in sel[0], its rank there in sel[1],
@@ -224,10 +265,9 @@ __global__ __launch_bounds__(1024) void sample_rows_kernel(const float* __restri
         auto window = [&](const uint32_t lo, const int sh, const unsigned need) {
             if (tid < 256) hist[tid] = 0u;
             __syncthreads();
-            for (int i = tid; i < V; i += 1024) {
-                const uint32_t d = kmax - order_key32(x[i]);
+            each([&](int, const uint32_t d) {
                 if (d >= lo && ((d - lo) >> sh) < 256u) atomicAdd(&hist[(d - lo) >> sh], 1u);
-            }
+            });
             __syncthreads();
             if (tid < 64) {
                 unsigned own = 0u;
@@ -271,16 +311,16 @@ __global__ __launch_bounds__(1024) void sample_rows_kernel(const float* __restri
     const uint32_t seed = (uint32_t)rng[2 * row], ctr = (uint32_t)rng[2 * row + 1];
     float best = -INFINITY;
     int besti = 0x7FFFFFFF;
-    for (int i = tid; i < V; i += 1024) {
-        const float v = x[i];
-        if (kmax - order_key32(v) > limit) continue;
+    each([&](const int i, const uint32_t d) {
+        if (d > limit) return;
+        const float v = from_order_key32(kmax - d);
         float sc = v;
         if (inv_temp > 0.0f) {
             const float u = ((float)(hash3(seed, ctr, (uint32_t)i) >> 8) + 0.5f) * (1.0f / 16777216.0f);
             sc = expf((v - mx) * inv_temp) / (-logf(u));
         }
         if (sc > best || (sc == best && i < besti)) { best = sc; besti = i; }
-    }
+    });
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) {
         const float ob = __shfl_xor(best, d);
@@ -374,8 +414,13 @@ int teal_sample_rows(const float* logits, int ld, int n_rows, int vocab, int top
                      int32_t* history, int history_len, void* stream) {
     if (!logits || !rng_state || !token_out || n_rows <= 0 || vocab <= 0 || (history && history_len <= 0)) return TEAL_ERR_ARG;
     if (ld < vocab) return TEAL_ERR_SHAPE;
-    hipLaunchKernelGGL(sample_rows_kernel, dim3(n_rows), dim3(1024), 0, reinterpret_cast<hipStream_t>(stream), logits, ld, vocab, top_k,
-                       temperature > 0.0f ? 1.0f / temperature : 0.0f, reinterpret_cast<unsigned long long*>(rng_state), token_out, pos_inout, history, history_len);
+    const bool vec = !(vocab & 3) && !(ld & 3) && aligned16(logits);
+#define TEAL_SR(P) hipLaunchKernelGGL((sample_rows_kernel<P>), dim3(n_rows), dim3(1024), 0, reinterpret_cast<hipStream_t>(stream), logits, ld, vocab, top_k, \
+                       temperature > 0.0f ? 1.0f / temperature : 0.0f, reinterpret_cast<unsigned long long*>(rng_state), token_out, pos_inout, history, history_len)
+    if (vec && vocab <= 4096 * 2) TEAL_SR(2);
+    else if (vec && vocab <= 4096 * 8) TEAL_SR(8);
+    else TEAL_SR(0);
+#undef TEAL_SR
     return launched();
 }
 

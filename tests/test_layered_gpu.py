@@ -161,6 +161,26 @@ def test_sampler_rows(V):
     assert (n / 1500 - p[0].cpu()).abs().max() < 0.05
 
 
+@pytest.mark.parametrize("V", [4, 4096, 8192, 8196, 32768, 32772])
+def test_sampler_rows_in_registers(V):
+    """rows that the sampler keeps in registers (aligned, whole 16 bytes) draw the same tokens as those it reads from memory on each pass, at the
+    ends of each register count; with ties, infinities, NaN and rows of one value"""
+    from teal_amd.kernels import layered as K
+    x = 3 * torch.randn(6, V, device=DEV)
+    x[1] = x[1].round()
+    x[2] = 0.25
+    x[3, ::3], x[3, 1::7] = float("nan"), -float("inf")
+    x[4, V // 2] = float("inf")
+    x[5] = float("nan")
+    loose = torch.empty(6, V + 1, device=DEV)[:, :V].copy_(x)
+    rng = torch.tensor([[11 + i, 0] for i in range(6)], device=DEV)
+    for temperature, k in ((0.0, None), (1.5, None), (0.8, 1), (0.8, min(200, V - 1)), (1e3, V - 1)):
+        for rep in range(3):
+            r2 = rng.clone()
+            assert torch.equal(K.sample_rows(x, rng, temperature, k), K.sample_rows(loose, r2, temperature, k)), (temperature, k)
+            assert torch.equal(rng, r2)
+
+
 # ---- the mixer alone: one key stands out ----------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("window", [1, 2, 63, 64, 65, 96, 300])
