@@ -17,7 +17,7 @@
 //
 // The attention kernels themselves (prompt_attention_*, step_attention_*) also serve grouped-query attention (teal_grouped.hip): `group`
 // query heads share a key / value head (prompts) or a segment of the cached row (single tokens), and scores can be soft-capped.
-#include "teal_prompt_attention.h"
+#include "teal_rows_core.h"
 
 namespace teal {
 
@@ -274,6 +274,91 @@ __global__ __launch_bounds__(256) void latent_step_query_kernel(const LatentStep
                 put(k.rank + 2 * i + 1, y);
             }
             for (int i = k.rank + k.rot + tid; i < a.ldq; i += 256) put(i, 0.0f);
+        }
+    }
+}
+
+// The same on the matrix cores, for up to sixteen tokens at once (their queries are 16-bit values: exact operands).  grid (heads * chunks
+// [+ 16 tokens' cache rows], batch / 16), four waves; a wave: 64 columns of the absorbed query, W_uk straight to its registers
+// (teal_rows_core.h), nothing shared.  Bound by latency: every load of 128 inputs is in flight at once.  16 tokens, 32 heads of 128, rank
+// 512: 7.6 -> 4.6 us (12 -> 5 with the cache rows, which one workgroup wrote for four tokens); 64 tokens: 19.6 -> 6.8
+template <bool BF16>
+__global__ __launch_bounds__(256) void latent_step_query_rows_kernel(const LatentStepArgs a, const int batch) {
+    constexpr int DT = BF16 ? TEAL_BF16 : TEAL_F16, FLIGHT = 4;
+    __shared__ float red[4];
+    const LatentRowArgs& k = a.kv;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
+    const int b0 = blockIdx.y * 16, nb = min(16, batch - b0);
+    const uint16_t* proj = reinterpret_cast<const uint16_t*>(k.proj) + (size_t)b0 * k.ldp;
+    const int extra = (int)blockIdx.x - k.heads * a.chunks;
+    if (extra >= 0) {
+        if (extra >= nb) return;
+        const int p = k.pos[b0 + extra];
+        const int row = page_row(a.table + (size_t)a.slot[b0 + extra] * a.max_pages, min(p, (a.max_pages << a.shift) - 1), a.shift);
+        latent_row<DT>(k, proj + (size_t)extra * k.ldp + k.kv0, p, reinterpret_cast<uint16_t*>(k.cache) + (size_t)row * k.ldc, red, tid);
+        return;
+    }
+    const int head = blockIdx.x / a.chunks, r0 = (blockIdx.x % a.chunks) * 256;
+    const uint16_t* qh = proj + head * (k.dim + k.rot);
+    uint16_t* out = reinterpret_cast<uint16_t*>(a.qcat) + ((size_t)b0 * k.heads + head) * 2 * a.ldq;  // token t: + t * heads * 2 * ldq
+    const int col = r0 + 64 * wave, wide = min(64, k.rank - col), ldb = 2 * k.rank, steps = k.dim / 32;
+    if (wide > 0) {
+        const RowsBuf buf[1] = {rows_buffer(reinterpret_cast<const uint16_t*>(a.uk) + (size_t)head * k.dim * k.rank + col, (size_t)(k.dim - 1) * ldb + 2 * wide)};
+        const uint32_t base = (uint32_t)(8 * g) * (uint32_t)ldb + 8u * (uint32_t)l16;
+        auto off = [&](const int s) { return 4 * l16 < wide && s < steps ? base + (uint32_t)s * 32u * (uint32_t)ldb : kRowsNowhere; };
+        const uint16_t* x = qh + (size_t)min(l16, nb - 1) * k.ldp + 8 * g;
+        RowsTile<4, 1> t[FLIGHT];
+        u32x4 xs[FLIGHT][1];
+        auto fetch = [&](const int i, const int s) {
+            rows_load<4, 1>(t[i], buf, off(s), ldb);
+            xs[i][0] = *reinterpret_cast<const u32x4*>(x + 32 * min(s, steps - 1));
+        };
+#pragma unroll
+        for (int i = 0; i < FLIGHT; ++i) fetch(i, i);
+        f32x4 acc[1][4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) acc[0][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < steps; s += FLIGHT)
+#pragma unroll
+            for (int i = 0; i < FLIGHT; ++i) {  // (steps past the last: zeros of W_uk)
+                rows_mfma<BF16, false, 1, 4, 1>(t[i], xs[i], acc);
+                if (s + FLIGHT < steps) fetch(i, s + FLIGHT + i);
+            }
+        // a lane holds token l16 and the columns 16 g .. 16 g + 15 of the wave's 64
+        if (l16 < nb && 16 * g < wide) {
+            uint16_t* o = out + (size_t)l16 * k.heads * 2 * a.ldq + col + 16 * g;
+            uint32_t hi[8], lo[8];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int f = 0; f < 4; f += 2) split16x2<BF16>(acc[0][f][i], acc[0][f + 1][i], hi[2 * i + f / 2], lo[2 * i + f / 2]);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                *reinterpret_cast<u32x4*>(o + 8 * h) = u32x4{hi[4 * h], hi[4 * h + 1], hi[4 * h + 2], hi[4 * h + 3]};
+                *reinterpret_cast<u32x4*>(o + a.ldq + 8 * h) = u32x4{lo[4 * h], lo[4 * h + 1], lo[4 * h + 2], lo[4 * h + 3]};
+            }
+        }
+    }
+    if (r0 != 0) return;
+    // the rotated part and the zeros behind it
+    const int pairs = k.rot / 2, tail = a.ldq - k.rank - k.rot, per = pairs + tail;
+    for (int i = tid; i < nb * per; i += 256) {
+        const int t = i / per, j = i - t * per;
+        uint16_t* o = out + (size_t)t * k.heads * 2 * a.ldq;
+        if (j >= pairs) {
+            const int c = k.rank + k.rot + j - pairs;
+            o[c] = o[a.ldq + c] = 0;
+            continue;
+        }
+        const uint16_t* qr = qh + (size_t)t * k.ldp + k.dim + 2 * j;
+        float v[2];
+        rotate_pair(bits_to_float(qr[0], BF16), bits_to_float(qr[1], BF16), k.pos[b0 + t], k.inv_freq[j], v[0], v[1]);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            uint32_t hi, lo;
+            split16<BF16>(v[e], hi, lo);
+            o[k.rank + 2 * j + e] = (uint16_t)hi;
+            o[a.ldq + k.rank + 2 * j + e] = (uint16_t)lo;
         }
     }
 }
@@ -685,6 +770,102 @@ __global__ __launch_bounds__(256) void latent_decode_merge_kernel(const LatentMe
     }
 }
 
+// The same on the matrix cores, four tokens to a workgroup of four waves: wave t merges token t's splits (a lane: two quads of the latent at a time,
+// eight splits in flight, no barrier), leaves the merged fp32 latent as three 16-bit parts that add up to it (24 bits: as exact
+// as the fp32 products above), and the product with W_uv has them as twelve rows.  A wave: 16 of the workgroup's 64 columns.  Bound by the partial results,
+// which a workgroup reads for its tokens and every 64 columns of the head.  32 heads, rank 512, vdim 128: 16 tokens
+// of 16 splits 17.3 -> 8.1 us, of 8 splits 14.5 -> 5.6; 64 tokens of 4 splits 49 -> 13.9
+template <bool BF16>
+__global__ __launch_bounds__(256) void latent_merge_rows_kernel(const LatentMergeArgs a, const int batch) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    uint16_t* op = reinterpret_cast<uint16_t*>(smem);  // [part * 4 + token][rank + 8]
+    constexpr int FLIGHT = 16;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4, head = blockIdx.y;
+    const int b0 = blockIdx.z * 4, nb = min(4, batch - b0), lo = a.rank + 8, steps = a.rank / 32;
+    const int stride = part_stride(a.rank), r4 = stride - 4, quads = a.rank / 4;
+    // W_uv: rows (columns of the result) past the head's last lie outside the buffer and read as zeros
+    const int v = blockIdx.x * 64 + wave * 16 + l16;
+    const RowsBuf buf = rows_buffer(reinterpret_cast<const uint16_t*>(a.uv) + (size_t)head * a.vdim * a.rank, (size_t)a.vdim * a.rank * 2);
+    const uint32_t base = v < a.vdim ? ((uint32_t)v * (uint32_t)a.rank + 8u * (uint32_t)g) * 2u : kRowsNowhere;
+    const float sink2 = a.sink ? bits_to_float(reinterpret_cast<const uint16_t*>(a.sink)[head], BF16) * kLog2e : -INFINITY;
+    const size_t vc = (size_t)head * a.vdim + min(v, a.vdim - 1);
+    const float gt = a.gate ? bits_to_float(reinterpret_cast<const uint16_t*>(a.gate)[(size_t)(b0 + min(g, nb - 1)) * a.ldg + vc], BF16) : 0.0f;
+    u32x4 w[FLIGHT];
+    auto weights = [&](const int s0) {
+#pragma unroll
+        for (int i = 0; i < FLIGHT; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b128(buf, (int)(s0 + i < steps ? base + 64u * (uint32_t)(v < a.vdim ? s0 + i : 0) : kRowsNowhere), 0, 0);
+    };
+    if (wave < nb) {
+        const float* part = a.part + ((size_t)(b0 + wave) * a.heads + head) * a.splits * stride;
+        f32x4 y[8][2];
+        auto load = [&](const int s0, const int q0) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) y[u][e] = *reinterpret_cast<const f32x4*>(part + (size_t)min(s0 + u, a.splits - 1) * stride + 4 * min(q0 + 64 * e + lane, quads - 1));
+        };
+        const float pm = lane < a.splits ? part[(size_t)lane * stride + r4] : -INFINITY, pl = lane < a.splits ? part[(size_t)lane * stride + r4 + 1] : 0.0f;
+        load(0, 0);
+        weights(0);
+        const float M = fmaxf(sink2, wave_max_f(pm));
+        const float pf = lane < a.splits ? exp2f(pm - M) : 0.0f;
+        const float inv = 1.0f / (wave_sum_f(pl * pf) + (a.sink ? exp2f(sink2 - M) : 0.0f));
+        for (int q0 = 0; q0 < quads; q0 += 128) {
+            f32x4 x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            for (int s0 = 0; s0 < a.splits; s0 += 8) {
+                if (s0 != 0 || q0 != 0) load(s0, q0);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const float f = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(pf), min(s0 + u, 63)));
+                    if (s0 + u < a.splits) {
+                        x[0] += y[u][0] * f;
+                        x[1] += y[u][1] * f;
+                    }
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int quad = q0 + 64 * e + lane;
+                if (quad >= quads) continue;
+                uint32_t pw[3][2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    float r[2] = {x[e][2 * j] * inv, x[e][2 * j + 1] * inv};
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) {
+                        const uint32_t c0 = float_to_bits<BF16>(r[0]), c1 = float_to_bits<BF16>(r[1]);
+                        pw[q][j] = c0 | (c1 << 16);
+                        r[0] = fabsf(r[0]) < INFINITY ? r[0] - bits_to_float(c0, BF16) : 0.0f;  // (an infinity or NaN is its first part)
+                        r[1] = fabsf(r[1]) < INFINITY ? r[1] - bits_to_float(c1, BF16) : 0.0f;
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x2*>(op + (4 * q + wave) * lo + 4 * quad) = u32x2{pw[q][0], pw[q][1]};
+            }
+        }
+    } else {
+        weights(0);
+    }
+    __syncthreads();
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    const uint16_t* xo = op + min(l16, 11) * lo + 8 * g;
+    for (int s0 = 0; s0 < steps; s0 += FLIGHT) {
+        if (s0) weights(s0);
+#pragma unroll
+        for (int i = 0; i < FLIGHT; ++i)
+            if (s0 + i < steps) acc = mfma16<BF16>(*reinterpret_cast<const u32x4*>(xo + 32 * (s0 + i)), w[i], acc);
+    }
+    // a lane holds column l16 and part g of the four tokens; lane group g finishes token g
+    float x = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float t = __shfl(acc[i], l16) + (__shfl(acc[i], l16 + 16) + __shfl(acc[i], l16 + 32));
+        x = g == i ? t : x;
+    }
+    if (a.gate) x *= sigmoid_f(gt);
+    if (g < nb && v < a.vdim) reinterpret_cast<uint16_t*>(a.y)[(size_t)(b0 + g) * a.ldy + vc] = (uint16_t)float_to_bits<BF16>(x);
+}
+
 // sizes the matrix-core form of the single-token attention covers
 inline bool step_on_matrix_cores(const int rank, const int ldq, const int dtype) {
     return (dtype == TEAL_BF16 || dtype == TEAL_F16) && rank <= 512 && ldq <= 32 * kStepKSteps;
@@ -781,6 +962,15 @@ int teal_latent_step_query(const void* proj, int ldp, int kv0, int batch, const 
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     return with_dtype(dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
+        if constexpr (DT != TEAL_F32) {
+            // (four tokens of 32 heads: 4.3 us against 3.8; six: 3.8 / 4.2; eight of 16 heads 3.9 / 6.5, six: the same)
+            if (batch > 4 && batch * heads >= 128 && !(dim & 31) && !(rank & 15) && !(rot & 7) && !(ldp & 7) && rank <= 8192 && aligned16(proj)) {
+                LatentStepArgs m = a;
+                m.chunks = (rank + 255) / 256;
+                hipLaunchKernelGGL((latent_step_query_rows_kernel<DT == TEAL_BF16>), dim3(heads * m.chunks + (kv0 >= 0 ? 16 : 0), (batch + 15) / 16), dim3(256), 0, st, m, batch);
+                return launched();
+            }
+        }
         const int nx = heads * chunks + (kv0 >= 0 ? 1 : 0);
         // (from eight tokens on a workgroup reads its weights once for four of them)
         if (batch >= 8 && dim <= 2048) hipLaunchKernelGGL((latent_step_query_kernel<DT, 4>), dim3(nx, (batch + 3) / 4), dim3(256), (size_t)4 * dim * sizeof(float), st, a, batch);
@@ -841,6 +1031,13 @@ int teal_latent_step_merge(const float* part, int splits, const void* uv, const 
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     return with_dtype(dtype, [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
+        if constexpr (DT != TEAL_F32) {
+            // (four tokens of 32 heads: 7.4 us against 8.7, three: the same; eight of 16 heads 7.4 / 16, six: 7.3 / 6.9)
+            if (batch >= 4 && batch * heads >= 128 && !(rank & 31) && rank <= 2048 && vdim <= 65536) {
+                hipLaunchKernelGGL((latent_merge_rows_kernel<DT == TEAL_BF16>), dim3((vdim + 63) / 64, heads, (batch + 3) / 4), dim3(256), (size_t)12 * (rank + 8) * 2, st, a, batch);
+                return launched();
+            }
+        }
         const int nx = (vdim + 31) / 32;
         if (batch >= 8 && rank <= 2048) hipLaunchKernelGGL((latent_decode_merge_kernel<DT, 4>), dim3(nx, heads, (batch + 3) / 4), dim3(256), (size_t)(4 * ((rank + 7) & ~7) + 1024) * sizeof(float), st, a, batch);
         else hipLaunchKernelGGL((latent_decode_merge_kernel<DT, 1>), dim3(nx, heads, batch), dim3(256), (size_t)(((rank + 7) & ~7) + 1024) * sizeof(float), st, a, batch);

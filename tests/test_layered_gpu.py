@@ -181,6 +181,60 @@ def test_sampler_rows_in_registers(V):
             assert torch.equal(rng, r2)
 
 
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("B,heads,dim,rot,vdim,rank", [(5, 26, 32, 8, 33, 32), (16, 8, 96, 0, 64, 272), (17, 8, 128, 64, 100, 512), (33, 4, 160, 16, 17, 544), (8, 16, 64, 24, 128, 2048)])
+def test_step_products_on_matrix_cores(B, heads, dim, rot, vdim, rank, dtype):
+    """the absorbed query and the merge of several tokens at the ends of their tiles (16 and 4 tokens, 64 columns, 4 and 16 steps), with sink and gate and splits
+    that got nothing.  The query's two halves: fp32 sums of exact products, then half a step of the low part; the merge: one rounding at the end, of fp32 sums
+    (every partial sum is below the sum of the sizes: 2^-19 of it)"""
+    from teal_amd.kernels import layered as K
+    from teal_amd import runtime
+    runtime.init()
+    torch.manual_seed(B)
+    r = lambda *s: torch.randn(*s, device=DEV)  # noqa: E731
+    ldq, nq, pages = -(-(rank + rot) // 32) * 32, heads * (dim + rot), 3
+    ldp = -(-(nq + rank + rot) // 8) * 8
+    proj, uk, uv = r(B, ldp).to(dtype), (0.1 * r(heads * dim, rank)).to(dtype), (0.1 * r(heads * vdim, rank)).to(dtype)
+    pos = torch.randint(0, 64 * pages, (B,), device=DEV, dtype=torch.int32)
+    slot, table = torch.randperm(B, device=DEV).int(), torch.randperm(B * pages, device=DEV).int().view(B, pages).contiguous()
+    inv, norm_w = torch.rand(max(1, rot // 2), device=DEV), r(rank).to(dtype)
+    qcat = torch.full((B, heads, 2, ldq), 7.0, device=DEV, dtype=dtype)
+    caches = [torch.full((B * pages * 64, ldq), 3.0, device=DEV, dtype=dtype) for _ in range(2)]
+    K.latent_step_query(proj, nq, pos, slot, table, 6, inv, norm_w, 1e-5, uk, heads, dim, rot, rank, caches[0], qcat)
+    one = torch.full((B, heads, 2, ldq), 9.0, device=DEV, dtype=dtype)
+    for b in range(B):  # token by token: the kernel of few tokens
+        K.latent_step_query(proj[b:b + 1], nq, pos[b:b + 1], slot[b:b + 1], table, 6, inv, norm_w, 1e-5, uk, heads, dim, rot, rank, caches[1], one[b:b + 1])
+    assert torch.equal(caches[0], caches[1])
+    assert torch.equal(qcat[..., rank:], one[..., rank:])
+    q = proj[:, :nq].view(B, heads, dim + rot)[..., :dim].double()
+    w = uk.double().view(heads, dim, rank)
+    want = torch.stack([q[:, h] @ w[h] for h in range(heads)], 1)
+    size = torch.stack([q[:, h].abs() @ w[h].abs() for h in range(heads)], 1)
+    got = qcat[..., :rank].double().sum(2)
+    step = 2.0 ** (-22 if dtype is F16 else -16)
+    assert ((got - want).abs() <= step * want.abs() + 2.0 ** -19 * size + 2.0 ** -24).all()
+    for splits in (1, 7, 20):
+        part = torch.full((B, heads, splits, (rank + 3) // 4 * 4 + 4), float("nan"), device=DEV)
+        part[..., :rank], part[..., -4], part[..., -3] = r(B, heads, splits, rank), 3 * r(B, heads, splits), 1 + torch.rand(B, heads, splits, device=DEV)
+        if splits > 1:
+            part[1, :, splits - 1, :rank], part[1, :, splits - 1, -4], part[1, :, splits - 1, -3] = 0.0, -float("inf"), 0.0
+        for sink, gate in ((None, None), (r(heads).to(dtype), r(B, heads * vdim + 5).to(dtype)[:, :heads * vdim])):
+            y = torch.full((B + 1, heads * vdim + 3), 7.0, device=DEV, dtype=dtype)
+            K.latent_step_merge(part, splits, uv, sink, gate, y[:B], B, heads, rank, vdim)
+            f = torch.exp2(part[..., -4].double())
+            den = (f * part[..., -3].double()).sum(-1) + (0 if sink is None else sink.double().exp())
+            o = (part[..., :rank].double() * f[..., None]).sum(2) / den[..., None]
+            big = (part[..., :rank].double().abs() * f[..., None]).sum(2) / den[..., None]
+            v = uv.double().view(heads, vdim, rank)
+            want = torch.stack([o[:, h] @ v[h].T for h in range(heads)], 1).reshape(B, -1)
+            size = torch.stack([big[:, h] @ v[h].abs().T for h in range(heads)], 1).reshape(B, -1)
+            if gate is not None:
+                want = want * gate.double().sigmoid()
+            err = (y[:B, :heads * vdim].double() - want).abs()
+            assert (err <= 2.0 ** (-11 if dtype is F16 else -8) * want.abs() + 2.0 ** -19 * size + 2.0 ** -24).all(), (splits, float(err.max()))
+            assert (y[B] == 7).all() and (y[:, heads * vdim:] == 7).all()
+
+
 # ---- the mixer alone: one key stands out ----------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("window", [1, 2, 63, 64, 65, 96, 300])
