@@ -367,7 +367,10 @@ __global__ __launch_bounds__(256) void latent_step_query_rows_kernel(const Laten
 // Single tokens, part 2: attention over the cached rows.  grid (splits, groups of up to 16 heads of one segment, batch), four waves.  A split takes a run of
 // 32-key tiles of the window.  Per tile: the waves share the score product by its inner dimension (both 16-key tiles, K steps
 // wave, wave + 4, ...; partial scores through LDS), then each wave owns a quarter of the latent's columns in the value product.
-// The tile's rows are staged transposed ([column][key]) for that product; the score product's operand comes straight from memory.
+// A tile's rows are read once, into the LDS as they lie: the score product takes eight elements of a row, the value product four rows of a
+// column (ds_read_b64_tr_b16); the next tile is on its way meanwhile.  Bound by what one CU can load: fetched twice, as operands and to be
+// stored transposed, 16 tokens of 32 heads at 1000 positions took 18.2 us, 14.0 now;
+// one token 7.4 and 6.0.
 // part [batch][heads][splits][part_stride(rank)] = {weighted latent (rank, padded to 4), max (log2 units), sum, -, -}.
 // ------------------------------------------------------------------------------------------------
 __host__ __device__ constexpr int part_stride(const int rank) { return ((rank + 3) & ~3) + 4; }
@@ -401,14 +404,18 @@ __device__ __forceinline__ KeyRange split_range(const int p, const int window, c
     return r;
 }
 
+// elements between the rows of a tile in the LDS: whole tiles of value columns, and 16 bytes more so that rows start in different banks
+__host__ __device__ inline int step_tile_row(const int ldq, const int rt) { return (ldq > rt * 16 ? ldq : rt * 16) + 8; }
+
 // TIED: the workgroups that hold the token's own key write its cache row before they read it (several of them, more than sixteen heads
 // to a key head: the same values).
 template <bool BF16, int RT, bool TIED, bool CAPPED>
 __global__ __launch_bounds__(256) void step_attention_kernel(const StepAttentionArgs a) {
-    constexpr int RPW = RT / 4, LT = 36;    // 16-column tiles per wave; row stride (keys) of the transposed tile
-    constexpr int KSW = kStepKSteps / 4, NI = (RT + 7) / 8;  // inner-dimension steps per wave; staging rounds
-    __shared__ __align__(16) uint16_t ct[RT * 16 * LT];
-    __shared__ __align__(16) float sp[4 * 2 * 64 * 4];       // partial scores, lane-major
+    constexpr int RPW = RT / 4, KSW = kStepKSteps / 4, NI = kStepKSteps / 2;  // 16-column tiles, inner-dimension steps per wave; pieces of a row per thread
+    __shared__ __align__(16) float sp[4 * 2 * 64 * 4];  // partial scores, lane-major
+    extern __shared__ __align__(16) unsigned char dyn[];
+    uint16_t* ct = reinterpret_cast<uint16_t*>(dyn);    // [32 keys][LD]
+    const int LD = step_tile_row(a.ldq, RT);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
     const int per = (a.group + 15) / 16, seg = blockIdx.y / per;
     const int split = blockIdx.x, h0 = seg * a.group + (blockIdx.y - seg * per) * 16, b = blockIdx.z;
@@ -426,10 +433,9 @@ __global__ __launch_bounds__(256) void step_attention_kernel(const StepAttention
         }
         return;
     }
-    extern __shared__ __align__(16) unsigned char dyn[];
     if constexpr (TIED) {
         constexpr int DT = BF16 ? TEAL_BF16 : TEAL_F16;
-        uint16_t* qs = reinterpret_cast<uint16_t*>(dyn);  // [nh][2][ldq]
+        uint16_t* qs = reinterpret_cast<uint16_t*>(dyn);  // [nh][2][ldq], where the first tile comes to lie later
         const uint16_t* proj = reinterpret_cast<const uint16_t*>(a.proj) + (size_t)b * a.ldp;
         for (int i = tid; i < nh * a.ldq; i += 256) {
             const int h = i / a.ldq, d = i - h * a.ldq;
@@ -465,29 +471,22 @@ __global__ __launch_bounds__(256) void step_attention_kernel(const StepAttention
     f32x4 o[RPW];
 #pragma unroll
     for (int r = 0; r < RPW; ++r) o[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int kp = tid & 15, cg = tid >> 4;  // staging: key pair, column group (8 columns, then every 128th)
-    u32x4 sx[NI], sy[NI], kf[KSW][2];        // the next tile: rows of keys 2 kp and 2 kp + 1; score operands
+    if constexpr (TIED) __syncthreads();  // (every wave has its queries)
+    // a thread's pieces: 16 bytes of row tid / 8, every eighth of the row.  Keys outside the share read as zeros (their rows may be another
+    // sequence's leftovers): they are requested outside the buffer
+    const int krow = tid >> 3, kc = tid & 7, ni = (a.ldq + 63) / 64;
+    u32x4 st[NI];
     auto fetch = [&](const int j0, const int base) {
-        // keys outside the share read as zero in the value product (their rows may be another sequence's leftovers)
-        const bool in0 = j0 + 2 * kp >= kr.lo && j0 + 2 * kp < kr.hi, in1 = j0 + 2 * kp + 1 >= kr.lo && j0 + 2 * kp + 1 < kr.hi;
-        const uint16_t* k0 = cache + (size_t)(base + l16) * a.ldc + g * 8;
+        const RowsBuf buf = rows_buffer(cache + (size_t)base * a.ldc, ((size_t)31 * a.ldc + a.ldq) * 2);
+        const uint32_t off = j0 + krow >= kr.lo && j0 + krow < kr.hi ? (uint32_t)krow * (uint32_t)(2 * a.ldc) + 16u * (uint32_t)kc : kRowsNowhere;
 #pragma unroll
-        for (int s = 0; s < KSW; ++s)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                kf[s][t] = u32x4{0u, 0u, 0u, 0u};
-                if (wave + 4 * s < ksteps) kf[s][t] = *reinterpret_cast<const u32x4*>(k0 + (size_t)t * 16 * a.ldc + (wave + 4 * s) * 32);
-            }
-        const uint16_t* r0 = cache + (size_t)(base + 2 * kp) * a.ldc;
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int c0 = (cg + 16 * i) * 8;
-            sx[i] = sy[i] = u32x4{0u, 0u, 0u, 0u};
-            if (c0 < RT * 16 && c0 < a.ldq) {
-                if (in0) sx[i] = *reinterpret_cast<const u32x4*>(r0 + c0);
-                if (in1) sy[i] = *reinterpret_cast<const u32x4*>(r0 + a.ldc + c0);
-            }
-        }
+        for (int i = 0; i < NI; ++i)
+            if (i < ni) st[i] = __builtin_amdgcn_raw_buffer_load_b128(buf, (int)(8 * (kc + 8 * i) < a.ldq ? off + (off == kRowsNowhere ? 0u : 128u * i) : kRowsNowhere), 0, 0);
+    };
+    auto lds_barrier = [&]() {  // (not __syncthreads(), which would wait for the next tile as well)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
     };
     const int jend = (kr.hi - 1) / 32 * 32;  // (a tile of 32 keys never crosses a page: pages hold 2^shift >= 32)
     int j0 = kr.lo / 32 * 32;
@@ -498,34 +497,28 @@ __global__ __launch_bounds__(256) void step_attention_kernel(const StepAttention
     }
     for (; j0 < kr.hi && kr.lo < kr.hi; j0 += 32) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int c0 = (cg + 16 * i) * 8;
-            if (c0 < RT * 16) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    *reinterpret_cast<uint32_t*>(ct + (c0 + 2 * j) * LT + 2 * kp) = (sx[i][j] & 0xFFFFu) | (sy[i][j] << 16);
-                    *reinterpret_cast<uint32_t*>(ct + (c0 + 2 * j + 1) * LT + 2 * kp) = (sx[i][j] >> 16) | (sy[i][j] & 0xFFFF0000u);
-                }
-            }
-        }
+        for (int i = 0; i < NI; ++i)
+            if (i < ni && 8 * (kc + 8 * i) < a.ldq) *reinterpret_cast<u32x4*>(ct + krow * LD + 8 * (kc + 8 * i)) = st[i];
+        lds_barrier();
         f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int q = 0; q < KSW; ++q)
             if (wave + 4 * q < ksteps) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    s[t] = mfma16<BF16>(kf[q][t], qf[q][0], s[t]);
-                    s[t] = mfma16<BF16>(kf[q][t], qf[q][1], s[t]);
+                    const u32x4 kf = *reinterpret_cast<const u32x4*>(ct + (t * 16 + l16) * LD + (wave + 4 * q) * 32 + 8 * g);
+                    s[t] = mfma16<BF16>(kf, qf[q][0], s[t]);
+                    s[t] = mfma16<BF16>(kf, qf[q][1], s[t]);
                 }
             }
 #pragma unroll
         for (int t = 0; t < 2; ++t) *reinterpret_cast<f32x4*>(sp + ((wave * 2 + t) * 64 + lane) * 4) = s[t];
-        __syncthreads();
         if (j0 + 32 < kr.hi) {
             const int base = next;
             next = page_row(table, min(j0 + 64, jend), a.shift);
             fetch(j0 + 32, base);
         }
+        lds_barrier();
         float mx = m;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -559,14 +552,14 @@ __global__ __launch_bounds__(256) void step_attention_kernel(const StepAttention
         l = l * al + ls;
 #pragma unroll
         for (int r = 0; r < RPW; ++r) {
-            const uint16_t* bp = ct + ((wave * RPW + r) * 16 + l16) * LT + g * 4;
-            const u32x2 w0 = *reinterpret_cast<const u32x2*>(bp), w1 = *reinterpret_cast<const u32x2*>(bp + 16);
+            const uint16_t* bp = ct + (g * 4 + (l16 >> 2)) * LD + (wave * RPW + r) * 16 + 4 * (l16 & 3);
+            const u32x2 w0 = lds_column4(bp), w1 = lds_column4(bp + 16 * LD);
             const u32x4 cf = {w0[0], w0[1], w1[0], w1[1]};
             o[r] *= al;
             o[r] = mfma16<BF16>(cf, ph, o[r]);
             o[r] = mfma16<BF16>(cf, pl, o[r]);
         }
-        __syncthreads();
+        lds_barrier();
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
@@ -872,8 +865,9 @@ inline bool step_on_matrix_cores(const int rank, const int ldq, const int dtype)
 }
 
 template <bool TIED>
-int launch_step(const StepAttentionArgs& a, const int batch, const size_t lds, const int dtype, hipStream_t st) {
+int launch_step(const StepAttentionArgs& a, const int batch, const size_t queries, const int dtype, hipStream_t st) {
     const int rt = a.rank <= 64 ? 4 : (a.rank <= 128 ? 8 : (a.rank <= 256 ? 16 : 32));
+    const size_t lds = std::max(queries, (size_t)32 * step_tile_row(a.ldq, rt) * 2);  // (<= 41472 bytes)
     const dim3 grid(a.splits, a.heads / a.group * ((a.group + 15) / 16), batch), block(256);
 #define TEAL_LD(BF, RT)                                                                                                \
     do {                                                                                                               \

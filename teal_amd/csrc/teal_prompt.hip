@@ -146,13 +146,6 @@ struct PromptAttention16Args {
     float scale2;         // scale in log2 units
 };
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-// ds_read_b64_tr_b16: of 16 lanes, lane i names the 8 bytes of row i / 4, columns 4 (i % 4) of a 4 x 16 block and receives column i
-__device__ __forceinline__ u32x2 lds_column4(const uint16_t* p) {
-    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
-}
-
 // Flash attention of 128 queries per workgroup over 64-row tiles of the cache as it is.  S^T = K Q^T and O^T = V^T P^T: a lane holds four
 // consecutive keys of one query after the first product, which is its operand of the second; V comes transposed out of the LDS
 // (ds_read_b64_tr_b16), so neither the weights nor V cross lanes or memory.  A wave takes 32 queries: at 16 every operand read from the

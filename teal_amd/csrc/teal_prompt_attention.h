@@ -15,6 +15,13 @@ __device__ __forceinline__ f32x4 mfma16(const u32x4 a, const u32x4 b, const f32x
     else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// ds_read_b64_tr_b16: of 16 lanes, lane i names the 8 bytes of row i / 4, columns 4 (i % 4) of a 4 x 16 block and receives column i
+__device__ __forceinline__ u32x2 lds_column4(const uint16_t* p) {
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
+}
+
 // 2^x of a non-positive x (v_exp_f32: one ulp; results below the normal range are zero)
 __device__ __forceinline__ float exp2_fast(const float x) { return __builtin_amdgcn_exp2f(x); }
 

@@ -435,7 +435,7 @@ class LatentAttention(nn.Module):
 
     def splits(self, batch: int, max_pos: int, dtype: torch.dtype) -> int:
         """workgroups the cached rows of one sequence are split over: one per CU in all (of a scalar kernel two), one 32-key tile each at least.
-        (Two per CU: attention and merge of 16 tokens at 1000 positions 27.6 us, one: 23.8; at 16 heads 22.5 and 18.4; 64 tokens at 250: 33.4, 32.8)"""
+        (Two per CU: attention and merge of 16 tokens at 1000 positions 21.4 us, one: 19.6; at 16 heads 20.1 and 16.2; 64 tokens at 250: 29.0, 28.6)"""
         groups, total = (self.a.heads, 512) if dtype == torch.float32 else (-(-self.a.heads // 16), 256)
         tiles = min(self.window, max_pos + 1) // 32 + 1
         return max(1, min(tiles, total // (batch * groups), self.MAX_SPLITS))
