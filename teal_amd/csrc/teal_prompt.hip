@@ -152,7 +152,6 @@ struct PromptAttention16Args {
 // LDS would serve one product, and the LDS, not the matrix cores, would be the limit (128 bytes per clock against 256 wanted).  The
 // running maximum is replaced only when a score exceeds it by kStaleMax (weights up to 2^8 then, which changes nothing in their relative
 // precision): rescaling the accumulators costs as much as a quarter of the products.
-constexpr float kStaleMax = 8.0f;
 template <bool BF16, int HD>
 __global__ __launch_bounds__(256, 2) void prompt_attention16_kernel(const PromptAttention16Args a) {
     constexpr int NQ = 2, BM = 128, BN = 64, KS = HD / 32, KT = BN / 16, VT = HD / 16, LK = HD + 8, LV = HD + 16, NT = 256, CH = HD / 8, NL = BN * CH / NT;

@@ -82,25 +82,26 @@ struct PromptAttentionArgs {
 // needs when the keys of two 16-key tiles are interleaved per lane group — the weights never cross lanes.  O^T = V^T P^T.
 // CAP: scores as they are; capped; capped and BOUNDED — a cap of at most kBoundedCap lets 2^score stand as it is (fp32 and bf16 reach
 // 2^127): no running maximum, nothing is rescaled.
+constexpr float kStaleMax = 8.0f;  // a running maximum is replaced only by scores that exceed it by this much (log2 units): weights up to 2^8 meanwhile
 enum { kCapNone = 0, kCapped = 1, kCapBounded = 2 };
 constexpr float kBoundedCap = 60.0f;  // 2^(60 log2(e)) = 2^86.6 per key
 
-template <bool BF16, int DQP, int DVP, int NQ, int BN, int NT, int CAP>
+// VEC: head sizes and row strides in whole 16 bytes.  Loads are unconditional then, at addresses clamped into the arrays, and what lies outside a head becomes
+// zero on the way to the LDS: under a condition a load is followed by the copy of its result, which waits for it on the spot.
+template <bool BF16, int DQP, int DVP, int NQ, int BN, int NT, int CAP, bool VEC>
 __global__ __launch_bounds__(NT) void prompt_attention_kernel(const PromptAttentionArgs a) {
     constexpr int KS = DQP / 32, KT = BN / 16, VT = DVP / 16, LK = DQP + 8, LV = BN + 8, BM = NT / 4 * NQ;
     __shared__ __align__(16) uint16_t ks[BN * LK];
     __shared__ __align__(16) uint16_t vs[DVP * LV];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
-    const int head = blockIdx.y;
-    const SeqSpan sq = a.seqs[a.tiles[2 * blockIdx.x]];
-    const int q_first = a.tiles[2 * blockIdx.x + 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g = lane >> 4;
+    const int tile = blockIdx.x / a.heads, head = blockIdx.x - tile * a.heads;  // (the heads of a tile start together: the tiles come longest first)
+    const SeqSpan sq = a.seqs[a.tiles[2 * tile]];
+    const int q_first = a.tiles[2 * tile + 1];
     const int dq = a.dim + a.rot;
     const uint16_t* kp = reinterpret_cast<const uint16_t*>(a.k);
     const uint16_t* krp = reinterpret_cast<const uint16_t*>(a.kr);
     const int kvh = head / a.group, kvs = a.heads / a.group * a.dim;  // key / value head; row stride of the keys
     const uint16_t* vp = reinterpret_cast<const uint16_t*>(a.vt) + (size_t)kvh * a.vdim * a.S;
-    const bool qvec = !(a.dim & 7) && !(a.rot & 7) && !(a.ldq & 7);
-    const bool kvec = !(a.dim & 7) && !(a.rot & 7);
 
     u32x4 qf[NQ][KS];
     int qpos[NQ];
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(NT) void prompt_attention_kernel(const PromptAttent
         for (int s = 0; s < KS; ++s) {
             const int d0 = s * 32 + g * 8;
             u32x4 w = {0u, 0u, 0u, 0u};
-            if (qvec) {
+            if constexpr (VEC) {
                 if (d0 < dq) w = *reinterpret_cast<const u32x4*>(src + d0);
             } else {
 #pragma unroll
@@ -144,11 +145,11 @@ __global__ __launch_bounds__(NT) void prompt_attention_kernel(const PromptAttent
         for (int i = 0; i < NK; ++i) {
             const int at = tid + NT * i, key = at / CK, d0 = (at % CK) * 8;
             const size_t row = (size_t)min(sq.k0 + kt + key, a.S - 1);
-            kreg[i] = u32x4{0u, 0u, 0u, 0u};
-            if (kvec) {
-                const uint16_t* src = d0 < a.dim ? kp + row * kvs + kvh * a.dim + d0 : krp + row * a.rot + d0 - a.dim;
-                if (d0 < dq) kreg[i] = *reinterpret_cast<const u32x4*>(src);
+            if constexpr (VEC) {
+                const int d = min(d0, dq - 8);
+                kreg[i] = *reinterpret_cast<const u32x4*>(d < a.dim ? kp + row * kvs + kvh * a.dim + d : krp + row * a.rot + d - a.dim);
             } else {
+                kreg[i] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const int d = d0 + j;
@@ -159,8 +160,7 @@ __global__ __launch_bounds__(NT) void prompt_attention_kernel(const PromptAttent
 #pragma unroll
         for (int i = 0; i < NV; ++i) {  // (S and every sequence's key base are multiples of 8: 16-byte loads)
             const int at = tid + NT * i, v = at / CV, c0 = (at % CV) * 8;
-            vreg[i] = u32x4{0u, 0u, 0u, 0u};
-            if (v < a.vdim && sq.k0 + kt + c0 < a.S) vreg[i] = *reinterpret_cast<const u32x4*>(vp + (size_t)v * a.S + sq.k0 + kt + c0);
+            vreg[i] = *reinterpret_cast<const u32x4*>(vp + (size_t)min(v, a.vdim - 1) * a.S + min(sq.k0 + kt + c0, a.S - 8));
         }
     };
     static_assert((BN * CK) % NT == 0 && (DVP * CV) % NT == 0, "whole staging rounds");
@@ -172,61 +172,77 @@ __global__ __launch_bounds__(NT) void prompt_attention_kernel(const PromptAttent
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < NK; ++i) {
-            const int at = tid + NT * i;
-            *reinterpret_cast<u32x4*>(ks + (at / CK) * LK + (at % CK) * 8) = kreg[i];
+            const int at = tid + NT * i, d0 = (at % CK) * 8;
+            *reinterpret_cast<u32x4*>(ks + (at / CK) * LK + d0) = !VEC || d0 < dq ? kreg[i] : u32x4{0u, 0u, 0u, 0u};
         }
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const int at = tid + NT * i;
-            *reinterpret_cast<u32x4*>(vs + (at / CV) * LV + (at % CV) * 8) = vreg[i];
+            const int at = tid + NT * i, c0 = (at % CV) * 8;
+            *reinterpret_cast<u32x4*>(vs + (at / CV) * LV + c0) = at / CV < a.vdim && sq.k0 + kt + c0 < a.S ? vreg[i] : u32x4{0u, 0u, 0u, 0u};
         }
         __syncthreads();
         if (sq.klo + kt + BN <= last) fetch(kt + BN);
         f32x4 s[NQ][KT];
 #pragma unroll
-        for (int t = 0; t < KT; ++t) {
+        for (int t = 0; t < KT; ++t)
 #pragma unroll
             for (int n = 0; n < NQ; ++n) s[n][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
 #pragma unroll
             for (int q = 0; q < KS; ++q) {
                 const u32x4 kf = *reinterpret_cast<const u32x4*>(ks + (t * 16 + l16) * LK + q * 32 + g * 8);
 #pragma unroll
                 for (int n = 0; n < NQ; ++n) s[n][t] = mfma16<BF16>(kf, qf[n][q], s[n][t]);
             }
-        }
         const int k_first = sq.klo + kt;
         // every query of the wave sees every key of the tile: no masks
         const bool open = whole && k_first + BN - 1 <= wq0 && k_first > wq0 + NQ * 16 - 1 - a.window;
-        float ms[NQ];
+        float ms[NQ], top[NQ];
+        bool grown = false;
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
-            float mx = m[n];
 #pragma unroll
             for (int t = 0; t < KT; ++t)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float v = s[n][t][r] * sc;
-                    if constexpr (CAP != kCapNone) v = soft_cap2(v, cl2);
-                    if (!open) {
-                        const int kpos = k_first + t * 16 + g * 4 + r;
-                        v = kpos <= qpos[n] && kpos > qpos[n] - a.window ? v : -INFINITY;
-                    }
-                    s[n][t][r] = v;
-                    if constexpr (CAP != kCapBounded) mx = fmaxf(mx, v);
+                    s[n][t][r] *= sc;
+                    if constexpr (CAP != kCapNone) s[n][t][r] = soft_cap2(s[n][t][r], cl2);
                 }
-            if constexpr (CAP == kCapBounded) {
-                ms[n] = 0.0f;
-            } else {
+            if (!open) {
+#pragma unroll
+                for (int t = 0; t < KT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int kpos = k_first + t * 16 + g * 4 + r;
+                        s[n][t][r] = kpos <= qpos[n] && kpos > qpos[n] - a.window ? s[n][t][r] : -INFINITY;
+                    }
+            }
+            float mx = -INFINITY;
+            if constexpr (CAP != kCapBounded) {
+#pragma unroll
+                for (int t = 0; t < KT; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[n][t][r]);
+            }
+            if constexpr (CAP != kCapBounded) {
                 mx = fmaxf(mx, __shfl_xor(mx, 16));
-                mx = fmaxf(mx, __shfl_xor(mx, 32));
-                ms[n] = mx == -INFINITY ? 0.0f : mx;
-                const float al = exp2_fast(m[n] - ms[n]);
-                m[n] = mx;
+                top[n] = fmaxf(mx, __shfl_xor(mx, 32));
+                grown = grown || top[n] > m[n] + kStaleMax;
+            }
+        }
+        if (CAP != kCapBounded && __any(grown)) {
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) {
+                const float now = fmaxf(m[n], top[n]), al = now == -INFINITY ? 1.0f : exp2_fast(m[n] - now);
+                m[n] = now;
                 l[n] *= al;
 #pragma unroll
                 for (int v = 0; v < VT; ++v) o[n][v] *= al;
             }
         }
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) ms[n] = CAP == kCapBounded || m[n] == -INFINITY ? 0.0f : m[n];
 #pragma unroll
         for (int b = 0; b < BN / 32; ++b) {
             u32x4 ph[NQ], pl[NQ];
@@ -289,25 +305,34 @@ __global__ __launch_bounds__(NT) void prompt_attention_kernel(const PromptAttent
     }
 }
 
-// queries per workgroup: NT / 4.  Head sizes: q . k up to 256; values up to 256, a workgroup of 512 threads 128
+// Queries per workgroup: NT / 4.  Head sizes: q . k up to 256; values up to 256, a workgroup of 512 threads 128.  Bound by the one workgroup a CU holds
+// (160 registers, eight waves): products, softmax and LDS reads of a tile hardly overlap.  3000 tokens of 3 to 5 requests, 32 heads: q . k 192
+// and values 128 134 -> 103 us, 128 and 128 with bounded scores 155 -> 89, of which the order of the tiles 25.  Tried and slower: 32 queries a
+// wave (twice the operands' use, 256 registers: 116 and 90), 64 queries a workgroup (142, 88), two workgroups a CU (spills: 138).
 template <bool BF16, int NT, int CAP>
 int launch_prompt(const PromptAttentionArgs& a, const int n_tiles, hipStream_t st) {
     const int dq = a.dim + a.rot;
-    const dim3 grid(n_tiles, a.heads), block(NT);
-#define TEAL_LP(DQ, DV, BN) do { hipLaunchKernelGGL((prompt_attention_kernel<BF16, DQ, DV, 1, BN, NT, CAP>), grid, block, 0, st, a); return launched(); } while (0)
+    if ((long long)a.heads * n_tiles > 0x7FFFFFFFll) return TEAL_ERR_SHAPE;
+    const dim3 grid(a.heads * n_tiles), block(NT);
+#define TEAL_LP(DQ, DV, BN, VEC) do { hipLaunchKernelGGL((prompt_attention_kernel<BF16, DQ, DV, 1, BN, NT, CAP, VEC>), grid, block, 0, st, a); return launched(); } while (0)
     // (capped scores come with values no wider than the keys: fewer combinations)
 #define TEAL_LP_V(DQ)                                                                                                   \
     do {                                                                                                               \
-        if constexpr (CAP == kCapNone || DQ == 64) { if (a.vdim <= 64) TEAL_LP(DQ, 64, 64); }                          \
-        if constexpr (CAP == kCapNone || DQ >= 128) { if (a.vdim <= 128) TEAL_LP(DQ, 128, 64); }                       \
-        if constexpr (NT == 256 && (CAP == kCapNone || DQ > 128)) TEAL_LP(DQ, 256, 32);                                \
+        if constexpr (CAP == kCapNone || DQ == 64) { if (a.vdim <= 64) TEAL_LP(DQ, 64, 64, true); }                    \
+        if constexpr (CAP == kCapNone || DQ >= 128) { if (a.vdim <= 128) TEAL_LP(DQ, 128, 64, true); }                 \
+        if constexpr (NT == 256 && (CAP == kCapNone || DQ > 128)) TEAL_LP(DQ, 256, 32, true);                            \
         return TEAL_ERR_SHAPE;                                                                                         \
     } while (0)
+    if (dq > 256) return TEAL_ERR_SHAPE;
+    if ((a.dim | a.rot | a.ldq) & 7) {  // any sizes, element by element
+        if (a.vdim <= 128) { if (dq <= 128) TEAL_LP(128, 128, 64, false); TEAL_LP(256, 128, 64, false); }
+        if constexpr (NT == 256) TEAL_LP(256, 256, 32, false);
+        return TEAL_ERR_SHAPE;
+    }
     if (dq <= 64) TEAL_LP_V(64);
     else if (dq <= 128) TEAL_LP_V(128);
     else if (dq <= 192) TEAL_LP_V(192);
-    else if (dq <= 256) TEAL_LP_V(256);
-    return TEAL_ERR_SHAPE;
+    TEAL_LP_V(256);
 #undef TEAL_LP_V
 #undef TEAL_LP
 }

@@ -309,8 +309,8 @@ class PromptBatch:
 
     def tiles(self, size: int) -> torch.Tensor:
         if size not in self._tiles:
-            # (last tiles first: with a causal mask they are the long ones)
-            t = [(i, q) for i, (_, n, _, _, _) in enumerate(self.spans) for q in range(0, n, size)][::-1]
+            # (those with most keys before them first: they take longest)
+            t = sorted(((i, q) for i, (_, n, _, _, _) in enumerate(self.spans) for q in range(0, n, size)), key=lambda t: -(self.spans[t[0]][2] + t[1]))
             self._tiles[size] = torch.tensor(t, dtype=torch.int32).to(self.device)
         return self._tiles[size]
 

@@ -235,6 +235,36 @@ def test_step_products_on_matrix_cores(B, heads, dim, rot, vdim, rank, dtype):
             assert (y[B] == 7).all() and (y[:, heads * vdim:] == 7).all()
 
 
+@pytest.mark.parametrize("dtype", [F16, BF16])
+@pytest.mark.parametrize("dim,rot,vdim,cap", [(128, 64, 128, None), (40, 8, 72, None), (64, 0, 64, 30.0), (136, 48, 200, None), (192, 64, 256, 80.0), (96, 16, 104, 20.0)])
+def test_prompt_attention_by_pieces_and_by_elements(dim, rot, vdim, cap, dtype):
+    """rows in whole 16 bytes are loaded in pieces, others element by element: the same products in the same order, so the same results.  Portions
+    that end inside a tile, a window, 64 and 128 queries to a workgroup; keys past a portion's last are never seen (they are NaN)"""
+    from teal_amd.kernels import layered as K
+    from teal_amd import runtime
+    runtime.init()
+    torch.manual_seed(dim)
+    heads, group = 4, 2
+    spans = [(0, 130, 70, 0, 0), (130, 1, 0, 256, 0), (131, 77, 0, 320, 0)]  # q0, nq, start, k0, klo (keys padded to 64 rows)
+    T, S = 208, 320 + 128
+    r = lambda *s: torch.randn(*s, device=DEV).to(dtype)  # noqa: E731
+    q, k, vt = r(T, heads * (dim + rot)), r(S, heads // group * dim), r(heads // group * vdim, S)
+    kr, gate, sink = (r(S, rot) if rot else None), r(T, heads * vdim), r(heads)
+    for q0, nq, start, k0, klo in spans:
+        end = k0 + start + nq - klo
+        k[end:k0 + -(-(end - k0) // 64) * 64] = float("nan")
+    loose = torch.empty(T, heads * (dim + rot) + 3, device=DEV, dtype=dtype)[:, :heads * (dim + rot)].copy_(q)
+    seqs = torch.tensor(spans, dtype=torch.int32, device=DEV)
+    for tile in (64, 128) if vdim <= 128 else (64,):
+        tiles = torch.tensor([(i, a) for i, s in enumerate(spans) for a in range(0, s[1], tile)], dtype=torch.int32, device=DEV)
+        for window in (1 << 30, 50):
+            out = [torch.zeros(T, heads * vdim, device=DEV, dtype=dtype) for _ in range(2)]
+            for y, x in zip(out, (q, loose)):
+                K.prompt_attention(x, k, kr, vt, sink, gate, y, seqs, tiles, tile, heads, dim, rot, vdim, window, (dim + rot) ** -0.5, group=group, softcap=cap)
+            assert out[0].isfinite().all() and out[0].abs().sum() > 0
+            assert torch.equal(out[0], out[1])
+
+
 # ---- the mixer alone: one key stands out ----------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("window", [1, 2, 63, 64, 65, 96, 300])
