@@ -5,9 +5,8 @@ sparsity.  One eager engine step over `--layers` distinct layers (so the weights
 with teal_set_phase_buffer / teal_set_phase_stride; per launch role the median over workgroups and layers of every stamp
 relative to the workgroup's entry, and the launch's extent (first entry -> last end over its workgroups).
 
-Stamps (thread 0, 100 MHz wall clock -> 10 ns): 1 arguments in registers, 2 producer done, 3 activations of the first pass
-ready, 4 list written, 5 every load of the pass issued, 6 first unit consumed, 7 pass done, 8 all passes done, 9 past the
-reduce barrier, 10 outputs stored."""
+Stamps (thread 0, 100 MHz wall clock -> 10 ns): 1 arguments in registers, 2 RMSNorm producer done, 3 activations in LDS, 5 first unit
+requested, 6 first unit consumed, 8 all units done, 9 past the reduce barrier, 10 outputs stored."""
 import argparse
 import os
 import sys
@@ -23,6 +22,7 @@ from teal_amd.gpt_fast.engine import DecodeEngine  # noqa: E402
 from teal_amd.quantize import quantize_model_int4  # noqa: E402
 
 ROW = 32
+STAMPS = [1, 2, 3, 5, 6, 8, 9, 10]
 
 
 def main():
@@ -63,7 +63,7 @@ def main():
         reps.append(buf.clone().cpu())
     roles = {"qkv (MODE 1)": 0, "wo (MODE 4)": 2, "gate|up (MODE 1)": 3, "down (MODE 2)": 4}
     print(f"{a.model} widths, int4-g{a.groupsize}, sparsity {a.sparsity}, {a.layers} layers, 5 eager steps; us after the workgroup's entry (median over workgroups x layers x steps)")
-    print("%-18s %5s %7s | %s" % ("launch", "wgs", "extent", "  ".join(f"[{i:2d}]" for i in range(1, 11))))
+    print("%-18s %5s %7s | %s" % ("launch", "wgs", "extent", "  ".join(f"[{i:2d}]" for i in STAMPS)))
     for name, off in roles.items():
         rel, ext, wgs = [], [], 0
         for b in reps:
@@ -72,7 +72,7 @@ def main():
                 live = r[:, 0] > 0
                 wgs = int(live.sum())
                 r = r[live]
-                rel.append((r[:, 1:11] - r[:, :1]).float() / 100.0)
+                rel.append((r[:, STAMPS] - r[:, :1]).float() / 100.0)
                 ext.append(float(r[:, 10].max() - r[:, 0].min()) / 100.0)
         rel = torch.cat(rel)
         med = rel.median(dim=0).values

@@ -1,4 +1,4 @@
-// teal_gemv_int4.hip — sparse GEMV over int4 group-quantised weights (second half).
+// teal_gemv_int4.hip — sparse GEMV over int4 group-quantised weights.
 //
 // The reference ships int4-g32/64/128 weight-only linears for its DENSE gpt-fast path only
 // (gpt-fast/quantize.py:58-162 group q-params / quantise / dequantise, :359-443 handler, :483-526 WeightOnlyInt4Linear,
@@ -38,7 +38,7 @@
 
 // Same rule as the 16-bit GEMV units (teal_gemv_kernel.h): no implicit contraction — every fused multiply-add below is an
 // explicit fmaf(), so the slab path and the rounded path, and this unit against the merge producers elsewhere, cannot drift
-// by an ulp when the compiler changes its mind (ADVICE round 3).
+// by an ulp when the compiler changes its mind.
 #pragma clang fp contract(off)
 #include <stdio.h>
 

@@ -5,7 +5,7 @@ reference's kernels/sparse_gemv.py, backed by hand-written HIP (libteal_hip.so) 
     qkv_gemv(x, weight, tq, tk, tv, sparsity_bin, kv_size)            <- kernels/sparse_gemv.py:196-237
     SparseGEMV / SparseQKVGEMV / DenseGEMV (torch.library wrappers)   <- kernels/sparse_gemv.py:249-307
 
-Differences, all deliberate (DESIGN.md):
+Differences, all deliberate:
   * no autotune / no first-call warm-up: launch geometry is a pure function of (Z, N, CU count);
     `sparsity_bin` is accepted and ignored (it only keyed the reference's autotune cache);
   * no separate zero-fill launch, no fp16 atomics: fp32 accumulate, one rounding, deterministic;
@@ -111,7 +111,7 @@ def sparse_gateup_silu(x: torch.Tensor, w1: torch.Tensor, w3: torch.Tensor, thre
 
 def qkv_gemv_int8(x: torch.Tensor, weight: torch.Tensor, scales: torch.Tensor, threshold_q: float, threshold_k: float,
                   threshold_v: float, sparsity_bin: int, kv_size: int) -> torch.Tensor:
-    """qkv_gemv on int8 weight-only-quantised weights (SURVEY §8(f) rank 4): weight int8 [N, Z] column-major
+    """qkv_gemv on int8 weight-only-quantised weights: weight int8 [N, Z] column-major
     (strides (1, ld)), scales [N] in x.dtype — the buffers of the reference's WeightOnlyInt8Linear
     (gpt-fast/quantize.py:339-357), re-laid like the fp16 path.  y = (sparse(x) @ weight.T) * scales with one
     rounding.  kv_size = 0: a single threshold (threshold_q)."""
@@ -146,7 +146,7 @@ def splitk_sparse_gemv_int8(x: torch.Tensor, weight: torch.Tensor, scales: torch
 
 def qkv_gemv_int4(x: torch.Tensor, weight: torch.Tensor, scales_and_zeros: torch.Tensor, threshold_q: float, threshold_k: float,
                   threshold_v: float, sparsity_bin: int, kv_size: int) -> torch.Tensor:
-    """qkv_gemv on int4 group-quantised weights (SURVEY 8(f) rank 4): weight = packed nibble image of W^T by row
+    """qkv_gemv on int4 group-quantised weights: weight = packed nibble image of W^T by row
     pairs, uint8 [Z / 2][N + pad] (quantize.pack_int4_colmajor); scales_and_zeros bf16 [Z / G][N][2] (the reference's tensor,
     gpt-fast/quantize.py:79-93).  y = sparse(x) @ dequant(W).T, fp32 accumulation, one rounding.  kv_size = 0: one threshold."""
     if not x.is_cuda or not weight.is_cuda or not scales_and_zeros.is_cuda:

@@ -1,7 +1,6 @@
 """Device-side plumbing shared by the ops: dtype codes, current stream, split-K workspace.
 
-PyTorch owns every buffer; the C ABI only borrows raw pointers for a stream-ordered launch
-(SURVEY §8(b) "Ownership").  The workspace (fp32 split-K slabs behind the library's header of arrival
+PyTorch owns every buffer; the C ABI only borrows raw pointers for a stream-ordered launch.  The workspace (fp32 split-K slabs behind the library's header of arrival
 counters and sampler scratch, teal_workspace_init) is one persistent tensor per (device, stream),
 allocated and prepared outside graph capture (the warm-up call every capture needs), so captured
 graphs see a static address and two streams never share a counter.
