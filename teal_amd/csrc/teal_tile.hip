@@ -156,14 +156,20 @@ extern "C" {
 int teal_tile_split(int M, int K, int N, int images, int slabs) {
     if (M <= 0 || K <= 0 || N <= 0 || images < 1 || images > 2 || (slabs && images > 1)) return TEAL_ERR_ARG;
     if ((K % kTileK) || (N & 15)) return 0;
-    // Where the library's product is the slower one (bf16, us library / this kernel, the reader's pass over the partial sums not counted): an image
-    // longer than wide, which the library does not split, 11008 -> 4096: 301 rows 90 / 47, 640: 106 / 74, 768: 103 / 91; a square one 4096 -> 4096:
-    // 128 rows 31 / 20, 200: 25 / 24; gate | up 4096 -> 2 x 11008: 128 rows 76 / 62, 320: 107 / 85, 384: 121 / 126.  A wide image with 16-bit
-    // results has too few workgroups here (4096 -> 12288: 128 rows 40 / 55, 640: 70 / 79), and so has a narrow pair
-    if (slabs ? M > (K >= 2 * N ? 640 : K >= N ? 192 : 0) : images == 1 || N < 8192 || M > 320) return 0;
     DeviceCtx* ctx = device_ctx();
     if (!ctx) return TEAL_ERR_NO_DEVICE;
-    return tile_plan(M, K, N, images, slabs != 0, ctx->num_cu).split;
+    const TilePlan plan = tile_plan(M, K, N, images, slabs != 0, ctx->num_cu);
+    // Where the library's product is the slower one (bf16, library / this kernel, with the norm that reads the result).  Partial sums: an image
+    // longer than wide, which the library does not split: up to 4096 columns 11008 -> 4096 1.17 to 2.5 at 65 to 640 rows, 16384 -> 4096 1.3 to 2.8,
+    // 8192 -> 2048 1.1 to 1.5, 5632 -> 2048 1.0 to 1.3; wider ones, whose column tiles leave the CUs unevenly filled, up to 160 rows (13824 -> 5120 1.07 to
+    // 1.5, 320 rows 1.08, 640 0.83; 28672 -> 8192 1.25 to 2.0, 384 rows 0.89).  Square images are the library's (4096: 96 rows 30 us / 27, 256: 29 / 33; 5120: 96 rows
+    // 34 / 41).  Gate and up apart (two calls of the library): from about a hundred rows on while one round of workgroups holds them
+    // all (4096 -> 2 x 11008: 80 rows 0.98, 128 to 320 1.23 to 1.36, 384, a second round, 0.97; 2048 -> 2 x 5632 1.2 to 1.65; 8192 -> 2 x 28672: 160 rows 1.21, 192 0.82);
+    // as one image the library has them in one call, which is faster (0.7 to 1.0)
+    if (slabs ? K < 2 * N || M > (N <= 4096 ? 640 : 160)
+              : images == 1 || N < 4096 || M <= 96 || M > 384 || (N + kTileCols - 1) / kTileCols * 2 * ((M + plan.rows - 1) / plan.rows) > ctx->num_cu)
+        return 0;
+    return plan.split;
 }
 
 int teal_tile_gemm(const void* x, int ldx, const void* w0, const void* w1, int ld, void* y0, void* y1, int ldy, float* slabs, int M, int K, int N, int dtype, void* stream) {

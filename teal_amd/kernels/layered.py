@@ -119,10 +119,6 @@ def gated_linear(lin, x, act: str, bias=None, tickets=None):
     N = lin.out_features // 2
     split = rows_split(x, w, True) if w is not None and not N & 63 else 0
     if split == 0:
-        w = rows_weight(lin) if x.shape[0] > ROWS_MAX else None
-        if w is not None and not N & 7 and tile_split(x, w[:N], 2):
-            gu = torch.empty(x.shape[0], 2 * N, device=x.device, dtype=x.dtype)
-            return gated_act(_tile_gemm(x, w, N, gu, gu[:, N:], w.data_ptr() + 2 * N), N, N, act, bias)
         return gated_act(lin(x), N, N, act, bias)
     y = torch.empty(x.shape[0], N, device=x.device, dtype=x.dtype)
     return _rows_gemm(x, w, N, split, ROWS_ROUNDED, tickets, y, w_up=w.data_ptr() + 2 * N, bias=None if bias is None else bias[:N], bias_up=None if bias is None else bias[N:],
